@@ -111,6 +111,9 @@ struct cache_entry {
     int seen = 0;
     hipGraph_t graph = nullptr;
     hipGraphExec_t exec = nullptr;
+    // a short graph's kernels in launch order (arguments owned by `graph`):
+    // launched one by one in place of an exec
+    std::vector<hipKernelNodeParams> direct;
     uint64_t last_use = 0;
 };
 
