@@ -2,22 +2,30 @@
 // batches (prefill, the audio prefix, N > 16) on the int8 matrix cores.
 // Call site: crates/openasr-core/src/ggml_runtime/cpu_graph.rs:3652-3686.
 //
-// A workgroup computes a 64-row x 64-column output tile: each of its four
-// waves owns 16 weight rows and all 64 columns (four 16-column MFMA groups),
-// so every weight fragment a wave loads feeds four column groups; where the
-// 64-column tiles would leave CUs idle, 32-column tiles (two groups). K is walked
-// in 256-element slices. A slice's activations (quants, scales and, for Q4_K,
-// the 32-element sums of the 64 columns) are staged in LDS, double-buffered:
-// right after a slice's barrier the workgroup requests the next slice's
-// activations and weights into registers, computes the current slice from
-// LDS, and stores the next slice into the other buffer at the top of the
-// next iteration -- one barrier a slice, the next slice's loads in flight
-// under this slice's arithmetic. A buffer is written again only after the
-// following barrier, which every wave reaches after its reads of it.
+// A workgroup computes a tile of 16 RW rows x 16 GRPS columns with RW KW
+// waves: K group kg (RW waves of 16 rows each, all columns) takes the
+// 256-element K slices kg, kg + KW, ..., so every weight fragment a wave
+// loads feeds GRPS column groups. A slice's activations (quants, scales and,
+// for Q4_K, the 32-element sums of the tile's columns) are staged in LDS by
+// its group, double-buffered: right after a round's barrier the workgroup
+// requests the next round's activations and weights into registers, computes
+// the current slices from LDS, and stores the next ones into the other
+// buffers at the top of the next iteration -- one barrier a round, the next
+// round's loads in flight under this round's arithmetic. A buffer is written
+// again only after the following barrier, which every wave reaches after its
+// reads of it. The groups' sums are added through LDS at the end.
 //
-// The arithmetic of a block unit is the GEMV's (mfma_units.h) and each lane
-// walks K in order, so the f64 block sums are the ones the CPU reference
-// forms and the bits equal the GEMV's.
+// What bounds it: with tiles for every CU the exact per-block epilogue on the
+// VALU (64 x 64 tiles, one group); with few tiles the round trip of a slice's
+// loads, K / 256 of them in turn (896 x 3584 x 78 Q8_0: 48 workgroups, 14
+// slices, 42 us), which the K groups take side by side. The launch picks the
+// form by the number of tiles.
+//
+// The arithmetic of a block unit is the GEMV's (mfma_units.h): exact block
+// terms, added in f64. A group walks its slices in order and the groups are
+// added in order; against one walk of K only the f64 rounding of the order
+// moves (2^-53 of a partial sum), which reaches the rounded f32 result about
+// once in 2^28 values.
 //
 // Tiles are dealt to the XCDs in contiguous runs (workgroup i runs on XCD
 // i % 8): XCD x takes tiles [x P, (x + 1) P), the column blocks of a row tile
@@ -54,27 +62,31 @@ struct mmq_args {
     const float * sub_bias[kGemmFloatMaxSubs + 1];
 };
 
-// the activations of one K slice of the tile's 64 columns
+// the activations of one K slice of the tile's 16 GRPS columns
+template <int GRPS>
 struct mmq_slice {
-    int8_t q[kMmqCols][256 + kMmqPad];
-    float d[8][kMmqCols];     // Q4_K: [0][col] the super-block scale; Q8_0: [block][col]
-    int16_t ss[kMmqCols][8];  // Q4_K: the 32-element sums
+    int8_t q[16 * GRPS][256 + kMmqPad];
+    float d[8][16 * GRPS];     // Q4_K: [0][col] the super-block scale; Q8_0: [block][col]
+    int16_t ss[16 * GRPS][8];  // Q4_K: the 32-element sums
 };
 
 // this thread's share of a slice, held in registers between its request and
 // its store into LDS
+template <int GRPS, int RW>
 struct mmq_act {
-    uint4 q[4];
+    uint4 q[4 * GRPS / RW];
     float d[4];
     uint4 ss;
 };
 
-template <int WT, int GRPS>
-__device__ __forceinline__ void mmq_act_load(const mmq_args & a, int n0, int ncol, int64_t ks, mmq_act & r) {
-    const int t = (int) threadIdx.x;
+// t: the thread's index among the 64 RW threads that stage the slice
+template <int WT, int GRPS, int RW>
+__device__ __forceinline__ void mmq_act_load(const mmq_args & a, int t, int n0, int ncol, int64_t ks,
+                                             mmq_act<GRPS, RW> & r) {
+    static_assert(GRPS <= 2 * RW, "a thread stages at most four scales");
 #pragma unroll
-    for (int u = 0; u < GRPS; u++) {
-        const int idx = t + 256 * u, col = idx >> 4, piece = idx & 15;
+    for (int u = 0; u < 4 * GRPS / RW; u++) {
+        const int idx = t + 64 * RW * u, col = idx >> 4, piece = idx & 15;
         const int64_t kk = ks * 256 + piece * 16;
         const bool ok = col < ncol && kk < a.K;
         // clamped address, unconditional load: masked when stored
@@ -100,13 +112,12 @@ __device__ __forceinline__ void mmq_act_load(const mmq_args & a, int n0, int nco
     }
 }
 
-template <int WT, int GRPS>
-__device__ __forceinline__ void mmq_act_store(const mmq_args & a, int ncol, int64_t ks, const mmq_act & r,
-                                              mmq_slice & S) {
-    const int t = (int) threadIdx.x;
+template <int WT, int GRPS, int RW>
+__device__ __forceinline__ void mmq_act_store(const mmq_args & a, int t, int ncol, int64_t ks,
+                                              const mmq_act<GRPS, RW> & r, mmq_slice<GRPS> & S) {
 #pragma unroll
-    for (int u = 0; u < GRPS; u++) {
-        const int idx = t + 256 * u, col = idx >> 4, piece = idx & 15;
+    for (int u = 0; u < 4 * GRPS / RW; u++) {
+        const int idx = t + 64 * RW * u, col = idx >> 4, piece = idx & 15;
         const bool ok = col < ncol && ks * 256 + piece * 16 < a.K;
         *(uint4 *) &S.q[col][piece * 16] = ok ? r.q[u] : make_uint4(0, 0, 0, 0);
     }
@@ -160,8 +171,8 @@ __device__ __forceinline__ void mmq_w_load(const mmq_args & a, const char * wrow
 }
 
 template <int GRPS>
-__device__ __forceinline__ void mmq_compute(const mmq_args & a, const mmq_slice & S, const mmq_w4 & w, int64_t ks,
-                                            int r, int g, double (&acc)[4][4]) {
+__device__ __forceinline__ void mmq_compute(const mmq_args & a, const mmq_slice<GRPS> & S, const mmq_w4 & w, int64_t ks,
+                                            int r, int g, double (&acc)[GRPS][4]) {
     (void) a;
     (void) ks;
 #pragma unroll
@@ -179,8 +190,8 @@ __device__ __forceinline__ void mmq_compute(const mmq_args & a, const mmq_slice 
 }
 
 template <int GRPS>
-__device__ __forceinline__ void mmq_compute(const mmq_args & a, const mmq_slice & S, const mmq_w8 & w, int64_t ks,
-                                            int r, int g, double (&acc)[4][4]) {
+__device__ __forceinline__ void mmq_compute(const mmq_args & a, const mmq_slice<GRPS> & S, const mmq_w8 & w, int64_t ks,
+                                            int r, int g, double (&acc)[GRPS][4]) {
     const int64_t nblk = a.K / 32;
     const int nb = (int) (nblk - ks * 8 < kQ8Group ? nblk - ks * 8 : kQ8Group);
     // block by block (each (row, column) sum still takes its blocks in order),
@@ -198,9 +209,37 @@ __device__ __forceinline__ void mmq_compute(const mmq_args & a, const mmq_slice 
     }
 }
 
-template <int WT, int GRPS>
-__global__ __launch_bounds__(256) void k_mmq(mmq_args a) {
-    __shared__ __align__(16) mmq_slice s_buf[2];
+// sibling products: row_tile's product becomes the launch's (a's weights, rows
+// and output), row_tile its tile; selected with constant indices (an index
+// into the argument arrays would put them in scratch memory)
+__device__ __forceinline__ void mmq_pick_product(mmq_args & a, int64_t & row_tile, int tile_rows) {
+    static_assert(kGemmFloatMaxSubs == 2, "product selection below");
+    if (a.nsub <= 0) return;
+    const int64_t r0 = row_tile * tile_rows;
+    int64_t base = 0, mend = a.sub_m0[1];
+    const char * sw = a.sub_W[0];
+    char * sd = a.sub_dst[0];
+    const float * sb = a.sub_bias[0];
+    if (r0 >= a.sub_m0[1]) {
+        base = a.sub_m0[1], mend = a.sub_m0[2];
+        sw = a.sub_W[1], sd = a.sub_dst[1], sb = a.sub_bias[1];
+    }
+    if (a.nsub >= 2 && r0 >= a.sub_m0[2]) {
+        base = a.sub_m0[2], mend = a.sub_m0[3];
+        sw = a.sub_W[2], sd = a.sub_dst[2], sb = a.sub_bias[2];
+    }
+    row_tile -= base / tile_rows;
+    a.M = mend - base;
+    a.W = sw;
+    a.dst = sd;
+    a.dst_nb1 = a.M * 4;  // each product's output is contiguous
+    a.epi.bias = sb;
+}
+
+template <int WT, int GRPS, int RW, int KW>
+__global__ __launch_bounds__(64 * RW * KW) void k_mmq(mmq_args a) {
+    constexpr int kRows = 16 * RW;
+    __shared__ __align__(16) mmq_slice<GRPS> s_buf[2][KW];
     using wregs = typename std::conditional<WT == GGML_TYPE_Q4_K, mmq_w4, mmq_w8>::type;
     // contiguous runs of tiles per XCD
     const int64_t id = blockIdx.x;
@@ -208,57 +247,62 @@ __global__ __launch_bounds__(256) void k_mmq(mmq_args a) {
     if (t >= a.tiles) return;  // before any barrier: the whole workgroup leaves
     int64_t row_tile = t / a.col_blocks;
     const int64_t col_block = t % a.col_blocks;
-    // sibling products: this tile's product, selected with constant indices
-    // (an index into the argument arrays would put them in scratch memory)
-    static_assert(kGemmFloatMaxSubs == 2, "product selection below");
-    if (a.nsub > 0) {
-        const int64_t r0 = row_tile * kMmqRows;
-        int64_t base = 0, mend = a.sub_m0[1];
-        const char * sw = a.sub_W[0];
-        char * sd = a.sub_dst[0];
-        const float * sb = a.sub_bias[0];
-        if (r0 >= a.sub_m0[1]) {
-            base = a.sub_m0[1], mend = a.sub_m0[2];
-            sw = a.sub_W[1], sd = a.sub_dst[1], sb = a.sub_bias[1];
-        }
-        if (a.nsub >= 2 && r0 >= a.sub_m0[2]) {
-            base = a.sub_m0[2], mend = a.sub_m0[3];
-            sw = a.sub_W[2], sd = a.sub_dst[2], sb = a.sub_bias[2];
-        }
-        row_tile -= base / kMmqRows;
-        a.M = mend - base;
-        a.W = sw;
-        a.dst = sd;
-        a.dst_nb1 = a.M * 4;  // each product's output is contiguous
-        a.epi.bias = sb;
-    }
+    mmq_pick_product(a, row_tile, kRows);
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int rw = wave % RW, kg = wave / RW, st = (int) threadIdx.x % (64 * RW);
     const int r = lane & 15, g = lane >> 4;
-    const int64_t row = row_tile * kMmqRows + wave * 16 + r;
-    const bool row_ok = row_tile * kMmqRows + wave * 16 < a.M;  // uniform per wave
+    const int64_t row = row_tile * kRows + rw * 16 + r;
+    const bool row_ok = row_tile * kRows + rw * 16 < a.M;  // uniform per wave
     const int n0 = (int) (col_block * 16 * GRPS);
     const int ncol = min(16 * GRPS, a.N - n0);
     const int64_t nks = (a.K + 255) / 256;
     const char * wrow = a.W + (row_ok ? row : 0) * a.row_bytes;
-    double acc[4][4];
+    double acc[GRPS][4];
 #pragma unroll
-    for (int grp = 0; grp < 4; grp++)
+    for (int grp = 0; grp < GRPS; grp++)
 #pragma unroll
         for (int i = 0; i < 4; i++) acc[grp][i] = 0.0;
-    mmq_act act;
+    mmq_act<GRPS, RW> act;
     wregs wn;
-    mmq_act_load<WT, GRPS>(a, n0, ncol, 0, act);
-    mmq_w_load(a, wrow, 0, g, wn);
-    for (int64_t ks = 0; ks < nks; ks++) {
-        mmq_slice & S = s_buf[ks & 1];
-        mmq_act_store<WT, GRPS>(a, ncol, ks, act, S);
+    // K group kg takes the slices kg, kg + KW, ...: every group runs the same
+    // number of rounds (barriers), the groups past the last slice idle
+    if (kg < nks) {
+        mmq_act_load<WT, GRPS, RW>(a, st, n0, ncol, kg, act);
+        mmq_w_load(a, wrow, kg, g, wn);
+    }
+    int buf = 0;
+    for (int64_t k0 = 0; k0 < nks; k0 += KW, buf ^= 1) {
+        const int64_t ks = k0 + kg;
+        mmq_slice<GRPS> & S = s_buf[buf][kg];
+        if (ks < nks) mmq_act_store<WT, GRPS, RW>(a, st, ncol, ks, act, S);
         const wregs w = wn;
         __syncthreads();
-        if (ks + 1 < nks) {
-            mmq_act_load<WT, GRPS>(a, n0, ncol, ks + 1, act);
-            mmq_w_load(a, wrow, ks + 1, g, wn);
+        if (ks + KW < nks) {
+            mmq_act_load<WT, GRPS, RW>(a, st, n0, ncol, ks + KW, act);
+            mmq_w_load(a, wrow, ks + KW, g, wn);
         }
-        if (row_ok) mmq_compute<GRPS>(a, S, w, ks, r, g, acc);
+        if (row_ok && ks < nks) mmq_compute<GRPS>(a, S, w, ks, r, g, acc);
+    }
+    if constexpr (KW > 1) {
+        // the groups' sums through the staging buffers, added in group order
+        double * s_acc = (double *) &s_buf[0][0];
+        static_assert(sizeof(s_buf) >= sizeof(double) * 256 * GRPS * RW * (KW - 1), "the staging buffers hold the sums");
+        __syncthreads();  // the last slices are read
+        if (kg > 0) {
+#pragma unroll
+            for (int grp = 0; grp < GRPS; grp++)
+#pragma unroll
+                for (int i = 0; i < 4; i++)
+                    s_acc[(((kg - 1) * RW + rw) * 4 * GRPS + 4 * grp + i) * 64 + lane] = acc[grp][i];
+        }
+        __syncthreads();
+        if (kg > 0) return;
+#pragma unroll
+        for (int k = 0; k < KW - 1; k++)
+#pragma unroll
+            for (int grp = 0; grp < GRPS; grp++)
+#pragma unroll
+                for (int i = 0; i < 4; i++) acc[grp][i] += s_acc[((k * RW + rw) * 4 * GRPS + 4 * grp + i) * 64 + lane];
     }
     if (!row_ok) return;
     // the adds, then (GELU_ERF) the lane's GELUs together, then the stores
@@ -335,22 +379,32 @@ void launch_mmq(int wtype, const char * W, int64_t row_bytes, int64_t M, int64_t
     a.N = (int) N;
     a.dst = dst;
     a.dst_nb1 = dst_nb1;
-    // 32-column tiles where 64-column tiles leave CUs idle (the audio
-    // encoder's 896-row projections over 390 positions: 98 -> 182 tiles)
-    const int64_t row_tiles = (m_all + kMmqRows - 1) / kMmqRows;
-    const bool narrow = N > 32 && row_tiles * ((N + kMmqCols - 1) / kMmqCols) < n_cu;
-    const int cols = narrow ? 32 : kMmqCols;
-    a.col_blocks = (N + cols - 1) / cols;
-    a.tiles = row_tiles * a.col_blocks;
-    a.per_xcd = (a.tiles + kMmqXcds - 1) / kMmqXcds;
-    const dim3 grid((unsigned) (a.per_xcd * kMmqXcds));
-    if (wtype == GGML_TYPE_Q4_K) {
-        if (narrow) hipLaunchKernelGGL((k_mmq<GGML_TYPE_Q4_K, 2>), grid, dim3(256), 0, stream, a);
-        else hipLaunchKernelGGL((k_mmq<GGML_TYPE_Q4_K, 4>), grid, dim3(256), 0, stream, a);
-    } else {
-        if (narrow) hipLaunchKernelGGL((k_mmq<GGML_TYPE_Q8_0, 2>), grid, dim3(256), 0, stream, a);
-        else hipLaunchKernelGGL((k_mmq<GGML_TYPE_Q8_0, 4>), grid, dim3(256), 0, stream, a);
-    }
+    auto go = [&](auto q4, auto q8, int grps, int rw, int kw) {
+        a.col_blocks = (N + 16 * grps - 1) / (16 * grps);
+        a.tiles = (m_all + 16 * rw - 1) / (16 * rw) * a.col_blocks;
+        a.per_xcd = (a.tiles + kMmqXcds - 1) / kMmqXcds;
+        const dim3 grid((unsigned) (a.per_xcd * kMmqXcds)), block((unsigned) (64 * rw * kw));
+        if (wtype == GGML_TYPE_Q4_K) hipLaunchKernelGGL(q4, grid, block, 0, stream, a);
+        else hipLaunchKernelGGL(q8, grid, block, 0, stream, a);
+    };
+    // The form by how many 64 x 64 tiles there are for the CUs: fewer tiles,
+    // more and smaller workgroups and more K groups in flight. Per call with
+    // the activation quantization and the wait, us, Q8_0 / Q4_K at 256 CUs
+    // (left: the form before, 64 x 32 tiles of one K group below 256 tiles):
+    //   28 tiles  896 x 3584 x 78    50.1 -> 28.0 / 32.2 -> 23.3 (16-row form; 32-row 31.8 / 24.3)
+    //   32 tiles  1024 x 3072 x 119  45.3 -> 25.9 / 30.2 -> 22.3
+    //   64 tiles  2048 x 6144 x 100  77.2 -> 48.5 / 46.8 -> 32.2 (32-row form, 4 groups; 16-row 51.2 / 33.1)
+    //   98 tiles  896 x 3584 x 390   52.1 -> 46.1 / 35.4 -> 32.8 (2 groups; 4 groups 49.8 / 35.7)
+    //   192 tiles 6144 x 2048 x 100  52.5 -> 45.9 / 31.0 -> 29.6
+    //   256 tiles 1024 x 2048 x 1000 49.6 -> 45.8 / 37.5 -> 35.7 (64 x 64 tiles, 2 groups)
+    //   392 tiles 3584 x 896 x 390   36.7 with one group, 39.0 with two
+    const int64_t tiles = (m_all + kMmqRows - 1) / kMmqRows * ((N + kMmqCols - 1) / kMmqCols);
+    const bool deep = K > 512;  // slices for four K groups (K = 384: two)
+    if (deep && 6 * tiles <= n_cu) go(k_mmq<GGML_TYPE_Q4_K, 2, 1, 4>, k_mmq<GGML_TYPE_Q8_0, 2, 1, 4>, 2, 1, 4);
+    else if (deep && 4 * tiles <= n_cu) go(k_mmq<GGML_TYPE_Q4_K, 2, 2, 4>, k_mmq<GGML_TYPE_Q8_0, 2, 2, 4>, 2, 2, 4);
+    else if (4 * tiles <= 3 * n_cu) go(k_mmq<GGML_TYPE_Q4_K, 2, 2, 2>, k_mmq<GGML_TYPE_Q8_0, 2, 2, 2>, 2, 2, 2);
+    else if (tiles <= n_cu) go(k_mmq<GGML_TYPE_Q4_K, 4, 4, 2>, k_mmq<GGML_TYPE_Q8_0, 4, 4, 2>, 4, 4, 2);
+    else go(k_mmq<GGML_TYPE_Q4_K, 4, 4, 1>, k_mmq<GGML_TYPE_Q8_0, 4, 4, 1>, 4, 4, 1);
 }
 
 }  // namespace mi355x

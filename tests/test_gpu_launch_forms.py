@@ -28,3 +28,38 @@ def test_short_graph_replays(ggml, gpu, n_ops):
         assert G.compute(gpu.backend) == 0
         assert np.array_equal(G.get(y).reshape(3, 1000), x * np.float32(f))
     G.free()
+
+
+# 64 x 64 tiles for 256 CUs: up to 42 (16-row form of four K groups), up to 64
+# (32 rows, four groups), up to 192 (two groups), up to 256 (64 x 64 tiles, two
+# groups), more (one group); at most two K slices take two groups
+@pytest.mark.parametrize("wname,m,k,n", [
+    ("q8_0", 16, 544, 65), ("q8_0", 1040, 1184, 97), ("q8_0", 896, 3584, 78), ("q8_0", 2048, 2336, 81),
+    ("q8_0", 2064, 320, 127), ("q8_0", 4080, 800, 129), ("q8_0", 6160, 544, 250), ("q8_0", 384, 384, 301),
+    ("q4_K", 16, 768, 65), ("q4_K", 1040, 1280, 97), ("q4_K", 2048, 2304, 81), ("q4_K", 4080, 768, 129),
+    ("q4_K", 6160, 512, 250),
+])
+def test_tile_gemm_forms(ggml, gpu, ref, wname, m, k, n):
+    """the exact tile GEMM's forms at ragged rows, columns and K slices: the
+    oracle's f32 values, but for sums on a rounding boundary"""
+    print(f"tile gemm {wname} {m} x {k} x {n}", flush=True)
+    wt = ggml.Q8_0 if wname == "q8_0" else ggml.Q4_K
+    wq = ggml.quantize(wt, ggml.synth_normal(3, m + k, m * k, 0.0, 0.02).reshape(m, k))
+    x = RNG.standard_normal((n, k)).astype(np.float32)
+    G = ggml.Graph()
+    X = G.new(ggml.F32, k, n)
+    W = G.new(wt, k, m, weight=True)
+    Y = G.lib.ggml_mul_mat(G.ctx, W, X)
+    G.lib.ggml_mul_mat_set_prec(Y, ggml.GGML_PREC_F32)
+    G.build(Y)
+    G.allocate(gpu.buft)
+    G.set(W, wq)
+    want = ref.mul_mat(wt, wq, m, k, x)
+    for _ in range(3):
+        G.set(X, x)
+        assert G.compute(gpu.backend) == 0
+        y = G.get(Y).reshape(n, m)
+        # f64 sums in another order: an f32 result moves only where its sum
+        # sits within 2^-50 of a rounding boundary, and then by one step
+        assert (y != want).mean() <= 1e-5 and np.abs(y - want).max() <= 2.0 ** -22 * np.abs(want).max()
+    G.free()
