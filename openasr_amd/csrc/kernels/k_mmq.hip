@@ -60,6 +60,7 @@ struct mmq_args {
     const char * sub_W[kGemmFloatMaxSubs + 1];
     char * sub_dst[kGemmFloatMaxSubs + 1];
     const float * sub_bias[kGemmFloatMaxSubs + 1];
+    bool sub_f16[kGemmFloatMaxSubs + 1];
 };
 
 // the activations of one K slice of the tile's 16 GRPS columns
@@ -220,20 +221,22 @@ __device__ __forceinline__ void mmq_pick_product(mmq_args & a, int64_t & row_til
     const char * sw = a.sub_W[0];
     char * sd = a.sub_dst[0];
     const float * sb = a.sub_bias[0];
+    bool sh = a.sub_f16[0];
     if (r0 >= a.sub_m0[1]) {
         base = a.sub_m0[1], mend = a.sub_m0[2];
-        sw = a.sub_W[1], sd = a.sub_dst[1], sb = a.sub_bias[1];
+        sw = a.sub_W[1], sd = a.sub_dst[1], sb = a.sub_bias[1], sh = a.sub_f16[1];
     }
     if (a.nsub >= 2 && r0 >= a.sub_m0[2]) {
         base = a.sub_m0[2], mend = a.sub_m0[3];
-        sw = a.sub_W[2], sd = a.sub_dst[2], sb = a.sub_bias[2];
+        sw = a.sub_W[2], sd = a.sub_dst[2], sb = a.sub_bias[2], sh = a.sub_f16[2];
     }
     row_tile -= base / tile_rows;
     a.M = mend - base;
     a.W = sw;
     a.dst = sd;
-    a.dst_nb1 = a.M * 4;  // each product's output is contiguous
+    a.dst_nb1 = a.M * (sh ? 2 : 4);  // each product's output is contiguous
     a.epi.bias = sb;
+    a.epi.f16_out = sh;
 }
 
 template <int WT, int GRPS, int RW, int KW>
@@ -326,7 +329,9 @@ __global__ __launch_bounds__(64 * RW * KW) void k_mmq(mmq_args a) {
 #pragma unroll
         for (int i = 0; i < 4; i++) {
             const int n = n0 + grp * 16 + 4 * g + i;
-            if (n < a.N) *(float *) (a.dst + (int64_t) n * a.dst_nb1 + row * 4) = o[grp * 4 + i];
+            if (n >= a.N) continue;
+            if (a.epi.f16_out) *(uint16_t *) (a.dst + (int64_t) n * a.dst_nb1 + row * 2) = float_to_half_bits(o[grp * 4 + i]);
+            else *(float *) (a.dst + (int64_t) n * a.dst_nb1 + row * 4) = o[grp * 4 + i];
         }
     }
 }
@@ -350,11 +355,13 @@ void launch_mmq(int wtype, const char * W, int64_t row_bytes, int64_t M, int64_t
         a.sub_W[0] = W;
         a.sub_dst[0] = dst;
         a.sub_bias[0] = epi.bias;
+        a.sub_f16[0] = epi.f16_out;
         for (int i = 0; i < nsub; i++) {
             a.sub_m0[i + 1] = m_all;
             a.sub_W[i + 1] = subs[i].a;
             a.sub_dst[i + 1] = subs[i].d;
             a.sub_bias[i + 1] = subs[i].bias;
+            a.sub_f16[i + 1] = subs[i].f16_out;
             m_all += subs[i].M;
         }
         a.sub_m0[nsub + 1] = m_all;
@@ -364,7 +371,9 @@ void launch_mmq(int wtype, const char * W, int64_t row_bytes, int64_t M, int64_t
         for (int i = 0; i < nsub; i++) {
             gemm_float_epi ei;
             ei.bias = subs[i].bias;
-            launch_mmq(wtype, subs[i].a, row_bytes, subs[i].M, K, act, N, subs[i].d, subs[i].M * 4, stream, n_cu, ei);
+            ei.f16_out = subs[i].f16_out;
+            launch_mmq(wtype, subs[i].a, row_bytes, subs[i].M, K, act, N, subs[i].d, subs[i].M * (ei.f16_out ? 2 : 4),
+                       stream, n_cu, ei);
         }
         return;
     }

@@ -495,6 +495,18 @@ struct planner {
         auto it = index.find(t);
         return it == index.end() || it->second < i;
     }
+    // the CPY of o (f32, contiguous) into a contiguous f16 tensor that the
+    // launch planned at node i may perform in o's place: o's only reader,
+    // of its shape, not over the columns x the launch's siblings share
+    const ggml_tensor * f16_copy_of(const ggml_tensor * o, int i, const ggml_tensor * x) const {
+        const ggml_tensor * c = sole_consumer(o, i + 1);
+        if (!c || c->op != GGML_OP_CPY || c->src[0] != o || c->type != GGML_TYPE_F16 || !is_contiguous(c) ||
+            !is_contiguous(o) || o->type != GGML_TYPE_F32 || !ready_before(c->src[1], i) || overlap(span_of(c), span_of(x)))
+            return nullptr;
+        for (int d = 0; d < 4; d++)
+            if (c->ne[d] != o->ne[d]) return nullptr;
+        return c;
+    }
     bool plan_norm(int i, const ggml_tensor * t);
     bool norm_rope_match(int i, const ggml_tensor * t, norm_rope_job & job, const ggml_tensor *& mul,
                          const ggml_tensor *& rope) const;
@@ -871,6 +883,11 @@ bool planner::plan_mul_mat(int i, const ggml_tensor * t) {
                 mepi.gelu_erf = true;
                 produced = u;
             }
+            const ggml_tensor * c = mmq16_ok ? nullptr : f16_copy_of(produced, i, x);
+            if (c && try_fold({c}, c, {}, nullptr)) {
+                mepi.f16_out = true;
+                produced = c;
+            }
             dst = (char *) produced->data;
             dst_nb1 = (int64_t) produced->nb[1];
         }
@@ -900,6 +917,19 @@ bool planner::plan_mul_mat(int i, const ggml_tensor * t) {
                 h2.nodes.push_back(u);
                 h2.reads.push_back(span_of(uw));
                 const ggml_tensor * out = u;
+                // the launch writing o, absorbing `node` and reading `extra`
+                auto sub_fold = [&](const ggml_tensor * node, const ggml_tensor * extra) {
+                    hoist h3 = h2;
+                    h3.nodes.push_back(node);
+                    if (extra) h3.reads.push_back(span_of(extra));
+                    hoist h4 = h3;
+                    h4.writes.push_back(span_of(node));
+                    if (!hoist_ok(i, h4)) return false;
+                    h2 = h3;
+                    sb.d = (char *) node->data;
+                    out = node;
+                    return true;
+                };
                 const ggml_tensor * ua = sole_consumer(u, j + 1);
                 if (ua && ua->op == GGML_OP_ADD && ua->type == GGML_TYPE_F32 && is_contiguous(ua)) {
                     const ggml_tensor * o = ua->src[0] == u ? ua->src[1] : ua->src[0];
@@ -907,23 +937,25 @@ bool planner::plan_mul_mat(int i, const ggml_tensor * t) {
                     for (int d = 0; d < 4 && same; d++) same = ua->ne[d] == u->ne[d];
                     const bool row = same && o->type == GGML_TYPE_F32 && is_contiguous(o) && o->ne[0] == u->ne[0] &&
                                      o->ne[1] * o->ne[2] * o->ne[3] == 1;
+                    // into an f16 tensor in one go where that holds: the f32
+                    // sums in between (and their memory) are then not touched
+                    const ggml_tensor * c = row && !mmq16_ok ? f16_copy_of(ua, i, x) : nullptr;
                     if (row && ready_before(o, i)) {
-                        hoist h3 = h2;
-                        h3.nodes.push_back(ua);
-                        h3.reads.push_back(span_of(o));
-                        h3.writes.push_back(span_of(ua));
-                        if (hoist_ok(i, h3)) {
+                        hoist keep = h2;
+                        h2.nodes.push_back(ua);
+                        if (c && sub_fold(c, o)) {
                             sb.bias = (const float *) o->data;
-                            sb.d = (char *) ua->data;
-                            out = ua;
-                            h2 = h3;
+                            sb.f16_out = true;
+                        } else {
+                            h2 = keep;
+                            if (sub_fold(ua, o)) sb.bias = (const float *) o->data;
                         }
                     }
+                } else if (const ggml_tensor * c = mmq16_ok ? nullptr : f16_copy_of(u, i, x)) {
+                    if (sub_fold(c, nullptr)) sb.f16_out = true;
                 }
-                if (out == u) {
-                    h2.writes.push_back(span_of(u));
-                    if (!hoist_ok(i, h2)) break;
-                }
+                h2.writes.push_back(span_of(out));
+                if (out == u && !hoist_ok(i, h2)) break;
                 h = h2;
                 msubs.push_back(sb);
                 msub_outs.push_back(out);
@@ -2106,7 +2138,9 @@ bool planner::plan() {
         }
         // a node other than MUL_MAT may overwrite memory the act region was
         // quantized from only through a view; be conservative for writers
-        if (t->op == GGML_OP_SET_ROWS || t->op == GGML_OP_CPY) act_src = nullptr;
+        // a write through a view may change the columns the act region holds
+        if ((t->op == GGML_OP_SET_ROWS || t->op == GGML_OP_CPY) && act_src && overlap(span_of(t), span_of(act_src)))
+            act_src = nullptr;
     }
     return true;
 }

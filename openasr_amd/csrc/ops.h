@@ -124,6 +124,7 @@ struct gemm_float_epi {
     bool gelu_erf = false;
     const float * bias_col = nullptr;
     int64_t perm_rows = 0;
+    bool f16_out = false;  // launch_mmq: the result rounded to f16 (dst_nb1 in bytes of it)
 };
 constexpr int kGemmFloatMaxSubs = 2;
 struct gemm_float_args {
@@ -165,6 +166,7 @@ struct gemm_float_sub {
     int64_t M = 0;
     char * d = nullptr;
     const float * bias = nullptr;
+    bool f16_out = false;  // launch_mmq: d is f16
 };
 bool gemm_float_supported(const tview & d, const tview & a, int atype, const tview & b, int btype);
 // how many K splits a launch of this product takes on n_cu CUs (1: none;

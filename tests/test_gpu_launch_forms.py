@@ -63,3 +63,55 @@ def test_tile_gemm_forms(ggml, gpu, ref, wname, m, k, n):
         # sits within 2^-50 of a rounding boundary, and then by one step
         assert (y != want).mean() <= 1e-5 and np.abs(y - want).max() <= 2.0 ** -22 * np.abs(want).max()
     G.free()
+
+
+@pytest.mark.parametrize("wname,m,k,n", [("q8_0", 384, 384, 301), ("q8_0", 64, 1056, 65), ("q4_K", 128, 512, 97)])
+@pytest.mark.parametrize("over_columns", [False, True])
+def test_products_into_f16_tensors(ggml, gpu, ref, wname, m, k, n, over_columns):
+    """products of the same columns copied into f16 tensors (the cross K/V of
+    an audio window), a bias on every second one: the bits of f16(product) and
+    f16(product + bias). over_columns: the first copy's destination lies over
+    the columns, so the later products read what it wrote."""
+    print(f"f16 products {wname} {m} x {k} x {n} over {over_columns}", flush=True)
+    wt = ggml.Q8_0 if wname == "q8_0" else ggml.Q4_K
+    G = ggml.Graph()
+    lib, ctx = G.lib, G.ctx
+    X = G.new(ggml.F32, k, n, weight=True)
+    W = [G.new(wt, k, m, weight=True) for _ in range(5)]
+    B = G.new(ggml.F32, m, weight=True)
+    C = [G.new(ggml.F16, m, n, weight=True) for _ in range(5)]
+    G.gf = lib.ggml_new_graph_custom(ctx, G.graph_size, False)
+    for i in range(5):
+        y = lib.ggml_mul_mat(ctx, W[i], X)
+        if i % 2:
+            y = lib.ggml_add(ctx, y, B)
+        lib.ggml_build_forward_expand(G.gf, lib.ggml_cpy(ctx, y, C[i]))
+    G.allocate(gpu.buft)
+    x = RNG.standard_normal((n, k)).astype(np.float32)
+    b = RNG.standard_normal(m).astype(np.float32)
+    wq = [ggml.quantize(wt, ggml.synth_normal(5, i, m * k, 0.0, 0.02).reshape(m, k)) for i in range(5)]
+    for t, q in zip(W, wq):
+        G.set(t, q)
+    G.set(B, b)
+    if over_columns:
+        ggml.tensor(C[0]).data = ggml.tensor(X).data
+        # the copies' nodes are views of their destinations
+        for i in range(lib.ggml_graph_n_nodes(G.gf)):
+            node = ggml.tensor(lib.ggml_graph_node(G.gf, i))
+            if node.view_src and node.src[1] == C[0]:
+                node.data = ggml.tensor(X).data
+    for _ in range(3):
+        G.set(X, x)
+        assert G.compute(gpu.backend) == 0
+        cols = x.copy()
+        for i in range(5):
+            y = ref.mul_mat(wt, wq[i], m, k, cols) + (b if i % 2 else np.float32(0))
+            want = y.astype(np.float16)
+            if over_columns and i == 0:
+                raw = cols.view(np.uint16).reshape(-1)
+                raw[:m * n] = want.view(np.uint16).reshape(-1)
+                cols = raw.view(np.float32).reshape(n, k)
+            else:
+                got = G.get(C[i], np.float16).reshape(n, m)
+                assert (got.view(np.uint16) != want.view(np.uint16)).mean() <= 1e-5
+    G.free()
