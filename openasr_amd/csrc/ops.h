@@ -219,6 +219,7 @@ struct fattn_args {
     // (k_fattn_mfma.hip, float tolerance) instead of the chunked definition
     int mfma;
     int mfma_split;  // KV splits of the matrix-core form (partials + combine when > 1)
+    bool mfma_merge;  // its splits merged in the workgroup instead
     // one query at the default precision: the workgroup form (k_fattn_dec.hip,
     // float tolerance); its KV splits (0: not used; > 1: partials + combine)
     int dec;

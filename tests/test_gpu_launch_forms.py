@@ -115,3 +115,49 @@ def test_products_into_f16_tensors(ggml, gpu, ref, wname, m, k, n, over_columns)
                 got = G.get(C[i], np.float16).reshape(n, m)
                 assert (got.view(np.uint16) != want.view(np.uint16)).mean() <= 1e-5
     G.free()
+
+
+# heads, kv heads, sequences, queries, span, live: split and combined (one
+# sequence), merged in the workgroup (a batch), one split, spans off the tile
+@pytest.mark.parametrize("d,hq,hkv,t,span,live", [
+    (128, 16, 8, 256, 512, 481), (128, 16, 8, 119, 1024, 1000), (64, 6, 6, 130, 600, 577), (128, 8, 1, 33, 300, 290),
+])
+@pytest.mark.parametrize("scale", [None, -0.11])
+def test_attention_batched_rows_keep_their_bits(ggml, gpu, d, hq, hkv, t, span, live, scale):
+    """a sequence's rows are the same bits in a batch, whose splits merge in
+    the workgroup, as alone, where they are written and combined; and f16
+    operands' distance from the 64-bit result"""
+    print(f"attention {d} {hq}/{hkv} {t} x {span} scale {scale}", flush=True)
+    S = 8
+    scale = d ** -0.5 if scale is None else scale
+    q = RNG.standard_normal((S, hq, t, d)).astype(np.float32)
+    k, v = (RNG.standard_normal((S, hkv, span, d)).astype(np.float16) for _ in range(2))
+    last = live - t + np.arange(t)
+    mask = np.where(np.arange(span)[None, :] <= last[:, None], 0.0, -np.inf).astype(np.float16)
+    mask[t // 2, 5:9] = -1.5  # neither open nor closed
+
+    def compute(seqs):
+        n = len(seqs)
+        G = ggml.Graph()
+        Q, K, V = G.new(ggml.F32, d, t, hq, n), G.new(ggml.F16, d, span, hkv, n), G.new(ggml.F16, d, span, hkv, n)
+        M = G.new(ggml.F16, span, t, 1, n)
+        y = G.lib.ggml_flash_attn_ext(G.ctx, Q, K, V, M, scale, 0.0, 0.0)
+        G.build(y)
+        G.allocate(gpu.buft)
+        for T, a in ((Q, q[seqs]), (K, k[seqs]), (V, v[seqs]), (M, np.broadcast_to(mask, (n, 1, t, span)))):
+            G.set(T, a)
+        assert G.compute(gpu.backend) == 0
+        out = G.get(y).reshape(n, t, hq, d)
+        G.free()
+        return out
+
+    batch = compute(list(range(S)))
+    for s in (0, 5):
+        assert np.array_equal(compute([s])[0], batch[s])
+    h = hq - 1
+    a = q[1, h].astype(np.float64) @ k[1, h // (hq // hkv)].astype(np.float64).T * scale + mask.astype(np.float64)
+    a = np.exp(a - a.max(1, keepdims=True))
+    want = (a / a.sum(1, keepdims=True)) @ v[1, h // (hq // hkv)].astype(np.float64)
+    # f16 queries move a score by at most its size times 2^-11 (|score| < 8
+    # here), f16 probabilities the result by 2^-11 of it
+    assert np.linalg.norm(batch[1, :, h] - want) <= 4 * 2.0 ** -11 * np.linalg.norm(want)
