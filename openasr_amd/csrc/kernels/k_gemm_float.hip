@@ -184,12 +184,12 @@ __device__ __forceinline__ void gf_mfma(const T (*sa)[kGfBK + PADE], const T (*s
 // wait for every load in flight.
 struct gf_raw {
     uint4 r[2];
-    bool ok;
+    uint32_t live;  // all ones, or 0 (a mask: a select per piece became an exec branch)
 };
 template <bool T16>
 __device__ __forceinline__ void gf_load_raw(const char * row, int64_t k0, int64_t K, bool live, gf_raw & v) {
-    v.ok = live && k0 < K;
-    const int64_t kc = v.ok ? k0 : 0;
+    v.live = live && k0 < K ? 0xFFFFFFFFu : 0u;
+    const int64_t kc = v.live ? k0 : 0;
     if constexpr (T16) {
         v.r[0] = *(const uint4 *) (row + 2 * kc);
     } else {
@@ -198,18 +198,22 @@ __device__ __forceinline__ void gf_load_raw(const char * row, int64_t k0, int64_
     }
 }
 
+__device__ __forceinline__ uint4 gf_and(const uint4 & v, uint32_t m) {
+    return make_uint4(v.x & m, v.y & m, v.z & m, v.w & m);
+}
+
 // a raw operand piece as eight f16 (T16 source: as is; f32: rounded to
 // nearest even) or eight f32 values, zeros when not live
 template <bool T16>
 __device__ __forceinline__ uint4 gf_as_f16(const gf_raw & v) {
-    if constexpr (T16) return v.ok ? v.r[0] : make_uint4(0, 0, 0, 0);
+    if constexpr (T16) return gf_and(v.r[0], v.live);
     const uint32_t f[8] = {v.r[0].x, v.r[0].y, v.r[0].z, v.r[0].w, v.r[1].x, v.r[1].y, v.r[1].z, v.r[1].w};
     uint32_t w[4];
 #pragma unroll
     for (int i = 0; i < 4; i++)
         w[i] = (uint32_t) float_to_half_bits(__uint_as_float(f[2 * i])) |
                ((uint32_t) float_to_half_bits(__uint_as_float(f[2 * i + 1])) << 16);
-    return v.ok ? make_uint4(w[0], w[1], w[2], w[3]) : make_uint4(0, 0, 0, 0);
+    return gf_and(make_uint4(w[0], w[1], w[2], w[3]), v.live);
 }
 template <bool T16>
 __device__ __forceinline__ void gf_as_f32(const gf_raw & v, uint4 & lo, uint4 & hi) {
@@ -227,7 +231,8 @@ __device__ __forceinline__ void gf_as_f32(const gf_raw & v, uint4 & lo, uint4 & 
         lo = v.r[0];
         hi = v.r[1];
     }
-    if (!v.ok) lo = hi = make_uint4(0, 0, 0, 0);
+    lo = gf_and(lo, v.live);
+    hi = gf_and(hi, v.live);
 }
 
 // a slab's pieces into LDS (sa, sb): f16 operands for an F16 src0 (the
@@ -262,7 +267,7 @@ __device__ __forceinline__ void gf_split8(const gf_raw & v, uint4 & hi, uint4 & 
         uint32_t hb[2], lb[2];
 #pragma unroll
         for (int e = 0; e < 2; e++) {
-            const float x = v.ok ? __uint_as_float(f[2 * i + e]) : 0.0f;
+            const float x = __uint_as_float(f[2 * i + e] & v.live);
             const __bf16 xh = (__bf16) x;
             const __bf16 xl = (__bf16) (x - (float) xh);
             hb[e] = __builtin_bit_cast(uint16_t, xh);
@@ -292,8 +297,15 @@ __global__ __launch_bounds__(kGfThreads) void k_gemm_float_v(gemm_float_args g) 
     __shared__ __align__(16) T sb[2][kGfBN][kGfBK + PADE];
     const int tid = (int) threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    int64_t m0 = (int64_t) blockIdx.x * kGfBM;
-    const int64_t n0 = (int64_t) blockIdx.y * kGfBN;
+    // the tile: contiguous runs of tiles a XCD; the column tiles of a row
+    // tile adjacent, then the row tiles, then the splits (or batches), so an
+    // XCD fetches a run of weight rows once, over its splits' part of K
+    const int64_t t = (int64_t) (blockIdx.x % 8) * g.per_xcd + blockIdx.x / 8;
+    if (t >= g.tiles) return;  // the grid's padding, before any barrier
+    const int64_t rt = t / g.col_blocks;
+    int64_t m0 = rt % g.row_blocks * kGfBM;
+    const int64_t n0 = t % g.col_blocks * kGfBN;
+    const int tz = (int) (rt / g.row_blocks);
     // sibling products: this tile's product (rows, weights, output, bias)
     // (selects with constant indices: an index into the argument arrays
     // would put the arguments in scratch memory)
@@ -318,8 +330,8 @@ __global__ __launch_bounds__(kGfThreads) void k_gemm_float_v(gemm_float_args g) 
         g.d_nb1 = g.M * 4;  // each product's output is contiguous
         g.epi.bias = sbias;
     }
-    // split: blockIdx.z is the split (one batch); else the batch
-    const int zb = g.splits > 1 ? 0 : (int) blockIdx.z, ks = g.splits > 1 ? (int) blockIdx.z : 0;
+    // tz: the split (one batch), or the batch
+    const int zb = g.splits > 1 ? 0 : tz, ks = g.splits > 1 ? tz : 0;
     const int i2 = zb % g.ne2, i3 = zb / g.ne2;
     const int64_t kb = (int64_t) ks * g.k_span;
     const int64_t K = g.splits > 1 ? (g.K - kb < g.k_span ? g.K - kb : g.k_span) : g.K;
@@ -447,8 +459,8 @@ __global__ __launch_bounds__(kGfThreads) void k_gemm_float_x3(gemm_float_args g)
     auto stage = [&](const gf_raw & a, const gf_raw & b, int buf) {
         uint4 hi, lo;
         if constexpr (ASPLIT) {
-            hi = a.ok ? a.r[0] : make_uint4(0, 0, 0, 0);
-            lo = a.ok ? a.r[1] : make_uint4(0, 0, 0, 0);
+            hi = gf_and(a.r[0], a.live);
+            lo = gf_and(a.r[1], a.live);
         } else {
             gf_split8(a, hi, lo);
         }
@@ -717,19 +729,23 @@ void launch_gemm_float(const tview & d, const tview & a, int atype, const tview 
     const dim3 grid((unsigned) ((m_all + kGfBM - 1) / kGfBM), (unsigned) ((g.N + kGfBN - 1) / kGfBN),
                     (unsigned) (g.splits > 1 ? g.splits : g.ne2 * g.ne3));
     if (aligned) {
-        if (g.a_f16 && g.b_f16) hipLaunchKernelGGL((k_gemm_float_v<true, true>), grid, dim3(kGfThreads), 0, s, g);
-        else if (g.a_f16) hipLaunchKernelGGL((k_gemm_float_v<true, false>), grid, dim3(kGfThreads), 0, s, g);
-        else if (g.b_f16) hipLaunchKernelGGL((k_gemm_float_v<false, true>), grid, dim3(kGfThreads), 0, s, g);
+        g.col_blocks = grid.y;
+        g.row_blocks = grid.x;
+        g.tiles = (int64_t) grid.x * grid.y * grid.z;
+        g.per_xcd = (g.tiles + 7) / 8;
+        const dim3 gv((unsigned) (g.per_xcd * 8));
+        if (g.a_f16 && g.b_f16) hipLaunchKernelGGL((k_gemm_float_v<true, true>), gv, dim3(kGfThreads), 0, s, g);
+        else if (g.a_f16) hipLaunchKernelGGL((k_gemm_float_v<true, false>), gv, dim3(kGfThreads), 0, s, g);
+        else if (g.b_f16) hipLaunchKernelGGL((k_gemm_float_v<false, true>), gv, dim3(kGfThreads), 0, s, g);
         else if (x3) {
             // one dim of tiles, dealt to the XCDs in contiguous runs
             g.tiles = (int64_t) grid.x * grid.y;
-            g.col_blocks = grid.y;
             g.per_xcd = (g.tiles + 7) / 8;
             const dim3 g1((unsigned) (g.per_xcd * 8), 1u, grid.z);
             if (a_split) hipLaunchKernelGGL(k_gemm_float_x3<true>, g1, dim3(kGfThreads), 0, s, g);
             else hipLaunchKernelGGL(k_gemm_float_x3<false>, g1, dim3(kGfThreads), 0, s, g);
         }
-        else hipLaunchKernelGGL((k_gemm_float_v<false, false>), grid, dim3(kGfThreads), 0, s, g);
+        else hipLaunchKernelGGL((k_gemm_float_v<false, false>), gv, dim3(kGfThreads), 0, s, g);
         if (g.splits > 1) {
             const int64_t blocks = std::min<int64_t>((g.M * g.N + 255) / 256, 4096);
             hipLaunchKernelGGL(k_gemm_float_reduce, dim3((unsigned) blocks), dim3(256), 0, s, g);
