@@ -161,3 +161,29 @@ def test_attention_batched_rows_keep_their_bits(ggml, gpu, d, hq, hkv, t, span, 
     # f16 queries move a score by at most its size times 2^-11 (|score| < 8
     # here), f16 probabilities the result by 2^-11 of it
     assert np.linalg.norm(batch[1, :, h] - want) <= 4 * 2.0 ** -11 * np.linalg.norm(want)
+
+
+def test_gelu_erf_against_math_erf(ggml, gpu):
+    """GELU_ERF over erf's whole bent range, both ends of it, zeros of either
+    sign, subnormals, infinities and NaN: the f32 rounding of math.erf, then the
+    op's own f32 steps"""
+    from math import erf
+    z = np.concatenate([np.linspace(-6.2, 6.2, 30001), np.geomspace(1e-45, 1e-2, 200), [0.0, -0.0, 5.65685, 5.656855,
+                        -5.65685, 1e30, np.inf, -np.inf, np.nan]]).astype(np.float32)
+    G = ggml.Graph()
+    X = G.new(ggml.F32, z.size)
+    E = G.lib.ggml_gelu_erf(G.ctx, X)
+    G.build(E)
+    G.allocate(gpu.buft)
+    G.set(X, z)
+    assert G.compute(gpu.backend) == 0
+    a = z * np.float32(0.70710678118654752440)
+    e = np.array([erf(float(v)) if np.isfinite(v) else np.sign(v) for v in a], np.float32)
+    with np.errstate(invalid="ignore"):
+        want = np.float32(0.5) * z * (np.float32(1) + e)
+    got = G.get(E)
+    same = (got.view(np.uint32) == want.view(np.uint32)) | (np.isnan(got) & np.isnan(want))
+    # math.erf itself is within one double ulp: the f32 roundings of the two
+    # differ once in ~2^27 values
+    assert same.all(), (z[~same], got[~same], want[~same])
+    G.free()
