@@ -106,6 +106,27 @@ __device__ __forceinline__ float fa_dot(const uint4 (&kr)[D / 8], const float * 
     return acc;
 }
 
+// the chains of two queries over one K row, interleaved (each in its order)
+template <int D>
+__device__ __forceinline__ void fa_dot2(const uint4 (&kr)[D / 8], const float * qa, const float * qb, float & a0,
+                                        float & a1) {
+    a0 = a1 = 0.0f;
+#pragma unroll
+    for (int u = 0; u < D / 8; u++) {
+        float kf[8];
+        unpack8(kr[u], kf);
+        const float4 x0 = *(const float4 *) (qa + 8 * u), x1 = *(const float4 *) (qa + 8 * u + 4);
+        const float4 y0 = *(const float4 *) (qb + 8 * u), y1 = *(const float4 *) (qb + 8 * u + 4);
+        const float xv[8] = {x0.x, x0.y, x0.z, x0.w, x1.x, x1.y, x1.z, x1.w};
+        const float yv[8] = {y0.x, y0.y, y0.z, y0.w, y1.x, y1.y, y1.z, y1.w};
+#pragma unroll
+        for (int i = 0; i < 8; i++) {
+            a0 = fmaf(kf[i], xv[i], a0);
+            a1 = fmaf(kf[i], yv[i], a1);
+        }
+    }
+}
+
 // the same chain with the query as f16 halves (its f16-rounded values), all
 // D/8 16-byte pieces requested before the first step: the chain then waits
 // on no LDS read (each step is one v_fma_mix_f32, both operands halves)
@@ -203,10 +224,20 @@ __device__ __forceinline__ void fa_scores(const fattn_args & a, const fa_tile & 
     uint4 kr[D / 8];
 #pragma unroll
     for (int u = 0; u < D / 8; u++) kr[u] = sm.k[p][u];
-    for (int r = wave; r < t.nrows; r += 4) {
-        const float acc = fa_dot<D>(kr, &sm.q[r][0]);
+    auto score = [&](int r, float acc) {
         const float mv = sm.mask[r / t.g][p];
         sm.s[r][p] = mv == -INFINITY ? -INFINITY : acc * a.scale + mv;
+    };
+    // two rows at a time: two chains in flight
+    for (int r = wave; r < t.nrows; r += 8) {
+        if (r + 4 < t.nrows) {
+            float a0, a1;
+            fa_dot2<D>(kr, &sm.q[r][0], &sm.q[r + 4][0], a0, a1);
+            score(r, a0);
+            score(r + 4, a1);
+        } else {
+            score(r, fa_dot<D>(kr, &sm.q[r][0]));
+        }
     }
 }
 
@@ -237,6 +268,24 @@ __device__ __forceinline__ void fa_pv_row(const fa_smem<D, R> & sm, int r, int d
 #pragma unroll
     for (int i = 0; i < DPT; i++) acc[i] = 0.0f;
     l = 0.0f;
+    if (__all(live == ~(uint64_t) 0)) {
+        // every row of the wave sees the whole chunk (all but the diagonal
+        // chunks of a causal prefill): the same steps without a branch a
+        // position, so the LDS reads run ahead of the chains
+#pragma unroll 4
+        for (int j = 0; j < kFaChunk; j += 4) {
+            const float4 p4 = *(const float4 *) &sm.s[r][j];
+            const float p[4] = {p4.x, p4.y, p4.z, p4.w};
+#pragma unroll
+            for (int u = 0; u < 4; u++) {
+                l = l + p[u];
+                const uint16_t * vr = vb + (j + u) * D;
+#pragma unroll
+                for (int i = 0; i < DPT; i++) acc[i] = fmaf(p[u], half_bits_to_float(vr[i]), acc[i]);
+            }
+        }
+        return;
+    }
     for (int j = 0; j < kFaChunk; j++) {
         if ((live >> j) & 1) {
             const float p = sm.s[r][j];
