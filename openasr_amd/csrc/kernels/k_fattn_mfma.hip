@@ -59,10 +59,21 @@ __device__ __forceinline__ fm_h8 fm_load8(const _Float16 * p) { return *(const f
 // entry's page); 3 4-byte rows -- four word loads the same way; 2 other
 // rows -- eight 2-byte loads, indexes clamped below n_kv. fm_mask_fix:
 // positions at or past n_kv become -inf.
+// MM 4: an f32 mask, rounded to f16 (what its CPY to an f16 mask would hold).
 template <int MM>
 __device__ __forceinline__ fm_u4 fm_mask_load(const uint16_t * row, int pos, int n_kv) {
     if constexpr (MM == 0) {
         return fm_u4{0, 0, 0, 0};
+    } else if constexpr (MM == 4) {
+        const float * f = (const float *) row;
+        float v[8];
+#pragma unroll
+        for (int j = 0; j < 8; j++) v[j] = f[min(pos + j, n_kv - 1)];
+        fm_u4 r;
+#pragma unroll
+        for (int j = 0; j < 4; j++)
+            r[j] = (uint32_t) float_to_half_bits(v[2 * j]) | ((uint32_t) float_to_half_bits(v[2 * j + 1]) << 16);
+        return r;
     } else if constexpr (MM == 1) {
         return *(const fm_u4 *) (row + min(pos, (n_kv - 1) & ~7));
     } else if constexpr (MM == 3) {
@@ -123,10 +134,15 @@ __device__ __forceinline__ void fm_merge(float & M, float & L, float m, float l,
 // the next live tile's K / V / mask are loaded into registers while the
 // current one is on the matrix cores.
 //
+// KV32: K and V are f32 (the encoders' head views of their projections),
+// staged rounded to f16 -- what a copy to f16 tensors ahead of the launch
+// would hold. With MM 4 the three conversion launches of an encoder layer go
+// (a 30 s encode: 11.8 us a layer).
+//
 // MG: the workgroup takes every split of its rows in turn and merges
 // their states in registers (fm_merge, in split order, what the combine
 // launch computes), writing no partials.
-template <int D, int MM, bool MG>
+template <int D, int MM, bool MG, bool KV32>
 __global__ __launch_bounds__(kFmThreads) void k_fattn_mfma(fattn_args a, float * __restrict__ out,
                                                            float * __restrict__ part) {
     constexpr int KS = D / 32;  // k steps of the score MFMA
@@ -169,7 +185,23 @@ __global__ __launch_bounds__(kFmThreads) void k_fattn_mfma(fattn_args a, float *
     const int span0 = t_begin * kFmTile;
 
     // registers for one tile in flight
-    fm_u4 kr[KLD], vr[VLD][2], mr[MLD];
+    constexpr int EW = KV32 ? 2 : 1;  // 16-byte loads an 8-element piece takes
+    fm_u4 kr[KLD][EW], vr[VLD][2][EW], mr[MLD];
+    // eight elements as f16
+    auto half8 = [](const fm_u4 (&r)[EW]) {
+        if constexpr (!KV32) {
+            return r[0];
+        } else {
+            fm_u4 h;
+#pragma unroll
+            for (int j = 0; j < 4; j++) {
+                const fm_u4 w = r[j >> 1];
+                h[j] = (uint32_t) float_to_half_bits(__uint_as_float(w[2 * (j & 1)])) |
+                       ((uint32_t) float_to_half_bits(__uint_as_float(w[2 * (j & 1) + 1])) << 16);
+            }
+            return h;
+        }
+    };
     auto issue = [&](int tile, bool masked) {
         const int p0 = tile * kFmTile;
         // every load unconditional (rows clamped into the span, the result
@@ -177,7 +209,9 @@ __global__ __launch_bounds__(kFmThreads) void k_fattn_mfma(fattn_args a, float *
 #pragma unroll
         for (int i = 0; i < KLD; i++) {
             const int e = tid + i * kFmThreads, p = e / PC, piece = e % PC;
-            kr[i] = *(const fm_u4 *) (kbase + (int64_t) min(p0 + p, a.n_kv - 1) * a.k_nb1 + 16 * piece);
+#pragma unroll
+            for (int w = 0; w < EW; w++)
+                kr[i][w] = *(const fm_u4 *) (kbase + (int64_t) min(p0 + p, a.n_kv - 1) * a.k_nb1 + 16 * (EW * piece + w));
         }
 #pragma unroll
         for (int i = 0; i < VLD; i++) {
@@ -185,7 +219,9 @@ __global__ __launch_bounds__(kFmThreads) void k_fattn_mfma(fattn_args a, float *
 #pragma unroll
             for (int h = 0; h < 2; h++) {
                 const int p = p0 + 2 * pair + h;
-                vr[i][h] = *(const fm_u4 *) (vbase + (int64_t) min(p, a.n_kv - 1) * a.v_nb1 + 16 * piece);
+#pragma unroll
+                for (int w = 0; w < EW; w++)
+                    vr[i][h][w] = *(const fm_u4 *) (vbase + (int64_t) min(p, a.n_kv - 1) * a.v_nb1 + 16 * (EW * piece + w));
             }
         }
         if (!masked) return;
@@ -283,12 +319,12 @@ __global__ __launch_bounds__(kFmThreads) void k_fattn_mfma(fattn_args a, float *
 #pragma unroll
         for (int i = 0; i < KLD; i++) {
             const int e = tid + i * kFmThreads, p = e / PC, piece = e % PC;
-            *(fm_u4 *) &s_k[p][8 * piece] = kr[i];
+            *(fm_u4 *) &s_k[p][8 * piece] = half8(kr[i]);
         }
 #pragma unroll
         for (int i = 0; i < VLD; i++) {
             const int e = tid + i * kFmThreads, pair = e % (kFmTile / 2), piece = e / (kFmTile / 2);
-            fm_u4 v0 = vr[i][0], v1 = vr[i][1];
+            fm_u4 v0 = half8(vr[i][0]), v1 = half8(vr[i][1]);
             if (masked) {  // an unmasked tile is open throughout
                 const int pr = rel + 2 * pair;  // even: both positions in one word
                 const uint32_t open = s_open[pr >> 5] >> (pr & 31);
@@ -557,6 +593,11 @@ bool fattn_mfma_supported(const fattn_args & a) {
            (!a.mask || a.m_ne2 == 1);
 }
 
+bool fattn_mfma_reads_f32(const fattn_args & a) {
+    // the 64-wide heads of the encoders (the staging registers double)
+    return a.mfma && a.d == 64 && !a.mfma_merge;
+}
+
 void launch_fattn_mfma(const fattn_args & a, void * scratch, float * out, hipStream_t s) {
     const int qb = fm_q_blocks(a);
     const bool merged = a.mfma_merge;
@@ -569,14 +610,24 @@ void launch_fattn_mfma(const fattn_args & a, void * scratch, float * out, hipStr
     auto form = [&](auto d, auto mg) {
         constexpr int D = decltype(d)::value;
         constexpr bool MG = decltype(mg)::value;
-        if (mm == 0) go(k_fattn_mfma<D, 0, MG>);
-        else if (mm == 1) go(k_fattn_mfma<D, 1, MG>);
-        else if (mm == 3) go(k_fattn_mfma<D, 3, MG>);
-        else go(k_fattn_mfma<D, 2, MG>);
+        if (mm == 0) go(k_fattn_mfma<D, 0, MG, false>);
+        else if (mm == 1) go(k_fattn_mfma<D, 1, MG, false>);
+        else if (mm == 3) go(k_fattn_mfma<D, 3, MG, false>);
+        else go(k_fattn_mfma<D, 2, MG, false>);
     };
     using d128 = std::integral_constant<int, 128>;
     using d64 = std::integral_constant<int, 64>;
-    if (a.d == 128 && merged) form(d128{}, std::true_type{});
+    if (a.mfma_kv32 || a.mfma_mask32) {
+        if (!fattn_mfma_reads_f32(a) || !a.mfma_kv32) {
+            note_hip_error(hipErrorInvalidValue);
+            return;
+        }
+        if (a.mfma_mask32) go(k_fattn_mfma<64, 4, false, true>);
+        else if (mm == 0) go(k_fattn_mfma<64, 0, false, true>);
+        else if (mm == 1) go(k_fattn_mfma<64, 1, false, true>);
+        else if (mm == 3) go(k_fattn_mfma<64, 3, false, true>);
+        else go(k_fattn_mfma<64, 2, false, true>);
+    } else if (a.d == 128 && merged) form(d128{}, std::true_type{});
     else if (a.d == 128) form(d128{}, std::false_type{});
     else if (merged) form(d64{}, std::true_type{});
     else form(d64{}, std::false_type{});

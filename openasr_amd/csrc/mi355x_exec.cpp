@@ -514,6 +514,9 @@ struct planner {
     bool plan_binary(const ggml_tensor * t);
     bool plan_fattn(int i, const ggml_tensor * t);
     bool make_fattn(const ggml_tensor * t, fattn_args & a);
+    bool fattn_kv32(const ggml_tensor * t, const fattn_args & a) const;
+    bool mask32_ok(int i, const ggml_tensor * c);
+    std::unordered_set<const ggml_tensor *> mask32;  // f16 masks not launched: their attention reads the f32 one
     void fattn_quant_out(int i, const ggml_tensor * t, fattn_args & a, const ggml_tensor *& view);
     bool plan_attn_step(int i, const ggml_tensor * t);
 };
@@ -1584,6 +1587,38 @@ void planner::fattn_quant_out(int i, const ggml_tensor * t, fattn_args & a, cons
     }
 }
 
+// the matrix-core attention t (planned as a) reads its f32 K and V itself:
+// both f32, on 16-byte boundaries, not under its output
+bool planner::fattn_kv32(const ggml_tensor * t, const fattn_args & a) const {
+    for (int k = 1; k <= 2; k++) {
+        tview f;
+        if (gqa_fold(t->src[k], f) || overlap(span_of(t), span_of(t->src[k]))) return false;
+    }
+    return t->src[1]->type == GGML_TYPE_F32 && t->src[2]->type == GGML_TYPE_F32 && fattn_mfma_reads_f32(a) &&
+           aligned16(a.k) && aligned16(a.v);
+}
+
+// c, planned at node i, is the CPY of an f32 mask that only a matrix-core
+// attention reads, which then reads the f32 mask itself and c is not launched:
+// nothing up to and with that attention writes the f32 mask's bytes
+bool planner::mask32_ok(int i, const ggml_tensor * c) {
+    const ggml_tensor * m = c->src[0];
+    if (c->type != GGML_TYPE_F16 || m->type != GGML_TYPE_F32 || (c->flags & GGML_TENSOR_FLAG_OUTPUT) ||
+        !is_contiguous(c) || !is_contiguous(m) || (c->src[1] && c->src[1] != c) || bypass.count(root_of(m)) || deferred.count(root_of(m)))
+        return false;
+    for (int d = 0; d < 4; d++)
+        if (c->ne[d] != m->ne[d]) return false;
+    const ggml_tensor * t = sole_consumer(c, i + 1);
+    fattn_args a;
+    if (!t || t->op != GGML_OP_FLASH_ATTN_EXT || t->src[3] != c || t->src[0] == c || !supports_op(be->dev, t)) return false;
+    if (no_fold.count(c) || !make_fattn(t, a) || !fattn_kv32(t, a)) return false;
+    const span sm = span_of(m);
+    for (int j = i + 1; j <= index.at(t); j++)
+        if (!is_view_op(cg->nodes[j]->op) && overlap(span_of(cg->nodes[j]), sm)) return false;
+    fold_reads.push_back({c, sm, i, index.at(t)});  // nor a launch moved there (validate)
+    return true;
+}
+
 bool planner::plan_fattn(int i, const ggml_tensor * t) {
     fattn_args a;
     if (!make_fattn(t, a)) return false;
@@ -1599,6 +1634,14 @@ bool planner::plan_fattn(int i, const ggml_tensor * t) {
     const size_t vbytes = v32 ? ((size_t) ggml_nelements(v) * 2 + 255) & ~(size_t) 255 : 0;
     gen_need = std::max(gen_need, part + kbytes + vbytes);
     const tview kv = make_view(k), vv = make_view(v);
+    a.mfma_kv32 = fattn_kv32(t, a);
+    if (mask32.count(t->src[3])) {
+        // the f32 mask in the place of its CPY (find_mask32's conditions)
+        const ggml_tensor * m = t->src[3]->src[0];
+        a.mfma_mask32 = true;
+        a.mask = (const char *) m->data;
+        a.m_nb1 = m->nb[1], a.m_nb2 = m->nb[2], a.m_nb3 = m->nb[3];
+    }
     backend_state * b = be;
     const int ncu = n_cu;
     float * out = (float *) t->data;
@@ -1629,7 +1672,9 @@ bool planner::plan_fattn(int i, const ggml_tensor * t) {
                 nb3 = d.nb[3];
             };
             char * g = gen_base(b);
-            if (k32 && v32 && !dense_f32(kv) && !dense_f32(vv)) {
+            if (la.mfma_kv32) {
+                // read as they are
+            } else if (k32 && v32 && !dense_f32(kv) && !dense_f32(vv)) {
                 // both strided head views: one launch for the two
                 tview dk = f16_dense(kv, g + part), dvw = f16_dense(vv, g + part + kbytes);
                 launch_copy_pair(dk, kv, dvw, vv, GGML_TYPE_F16, GGML_TYPE_F32, s, ncu);
@@ -2063,6 +2108,11 @@ bool planner::plan() {
                 if (naive_jobs.count(t)) {
                     if (!plan_naive(i, t)) return false;
                     continue;
+                }
+                if (t->op == GGML_OP_CPY && mask32_ok(i, t)) {
+                    mask32.insert(t);
+                    deferred[t] = t;
+                    break;
                 }
                 const ggml_tensor * dst = t;
                 const tview dv = make_view(dst), av = view_of(t->src[0]);

@@ -187,3 +187,56 @@ def test_gelu_erf_against_math_erf(ggml, gpu):
     # differ once in ~2^27 values
     assert same.all(), (z[~same], got[~same], want[~same])
     G.free()
+
+
+@pytest.mark.parametrize("heads,t,n", [(14, 390, 1), (3, 97, 1), (2, 64, 2), (1, 2, 3)])
+@pytest.mark.parametrize("overwritten", [False, True])
+def test_attention_over_f32_keys_and_mask(ggml, gpu, heads, t, n, overwritten):
+    """an encoder's attention over strided f32 K / V head views and a mask cast
+    from f32: the bits of the same attention over f16 tensors holding their
+    roundings. overwritten: the f32 mask changes between its cast and the
+    attention, which must not see it"""
+    d = 64
+    print(f"f32 attention {heads} x {t} x {n} overwritten {overwritten}", flush=True)
+    q, k, v = (RNG.standard_normal((n, t, heads, d)).astype(np.float32) for _ in range(3))
+    mask = RNG.standard_normal((n, 1, t, t)).astype(np.float32)
+    mask[RNG.random(mask.shape) < 0.3] = -np.inf
+    mask[..., 0] = 0.0
+    for kind in ("zero", "mixed"):
+        m = np.zeros_like(mask) if kind == "zero" else mask
+        outs = []
+        for f32 in (True, False):
+            G = ggml.Graph()
+            lib, ctx = G.lib, G.ctx
+            head = lambda x: lib.ggml_permute(ctx, x, 0, 2, 1, 3)  # noqa: E731
+            Q = G.new(ggml.F32, d, heads, t, n)
+            G.gf = lib.ggml_new_graph_custom(ctx, G.graph_size, False)
+            if f32:
+                K, V = (G.new(ggml.F32, d, heads, t, n) for _ in range(2))
+                M = G.new(ggml.F32, t, t, 1, n)
+                m16 = lib.ggml_cast(ctx, M, ggml.F16)
+                lib.ggml_build_forward_expand(G.gf, m16)
+                if overwritten:
+                    O = G.new(ggml.F32, t, t, 1, n)
+                    lib.ggml_build_forward_expand(G.gf, lib.ggml_cpy(ctx, O, M))
+                y = lib.ggml_flash_attn_ext(ctx, head(Q), head(K), head(V), m16, d ** -0.5, 0.0, 0.0)
+            else:
+                K, V = (G.new(ggml.F16, d, t, heads, n) for _ in range(2))
+                M = G.new(ggml.F16, t, t, 1, n)
+                y = lib.ggml_flash_attn_ext(ctx, head(Q), K, V, M, d ** -0.5, 0.0, 0.0)
+            lib.ggml_set_output(y)
+            lib.ggml_build_forward_expand(G.gf, y)
+            G.allocate(gpu.buft)
+            for _ in range(2):
+                G.set(Q, q)
+                if f32:
+                    G.set(K, k), G.set(V, v), G.set(M, m)
+                    if overwritten:
+                        G.set(O, np.full_like(m, 3.0) * np.arange(t, dtype=np.float32))
+                else:
+                    G.set(K, k.astype(np.float16).transpose(0, 2, 1, 3)), G.set(V, v.astype(np.float16).transpose(0, 2, 1, 3))
+                    G.set(M, m.astype(np.float16))
+                assert G.compute(gpu.backend) == 0
+            outs.append(G.get(y))
+            G.free()
+        assert np.array_equal(outs[0], outs[1]) and np.isfinite(outs[0]).all()
