@@ -240,3 +240,72 @@ def test_attention_over_f32_keys_and_mask(ggml, gpu, heads, t, n, overwritten):
             outs.append(G.get(y))
             G.free()
         assert np.array_equal(outs[0], outs[1]) and np.isfinite(outs[0]).all()
+
+
+# rows of a multiple of eight elements on 16 bytes take eight a thread; others
+# (an odd width, an offset view) one
+@pytest.mark.parametrize("d,heads,t,n,span,skip", [(128, 8, 256, 8, 300, 0), (64, 3, 7, 2, 9, 0), (8, 1, 1, 1, 3, 0),
+                                                   (20, 3, 5, 2, 8, 0), (64, 3, 7, 2, 9, 1)])
+@pytest.mark.parametrize("i64", [False, True])
+def test_set_rows_widths(ggml, gpu, d, heads, t, n, span, skip, i64):
+    """f32 rows [d, t, heads, n] of a strided source into an f16 cache at
+    per-sequence rows: f16 roundings at those rows, the other rows untouched"""
+    print(f"set_rows {d} x {t} x {heads} x {n} skip {skip}", flush=True)
+    G = ggml.Graph()
+    lib, ctx = G.lib, G.ctx
+    X = G.new(ggml.F32, d + 4 * skip, heads, t, n)
+    I = G.new(ggml.I64 if i64 else ggml.I32, t, 1, n)
+    C = G.new(ggml.F16, d, span, heads, n, weight=True)
+    src = lib.ggml_permute(ctx, X, 0, 2, 1, 3)
+    if skip:
+        # the last d of d + 4 elements, from 4 bytes past a 16-byte boundary
+        src = lib.ggml_permute(ctx, lib.ggml_view_4d(ctx, X, d, heads, t, n, 4 * (d + 4), 4 * (d + 4) * heads,
+                                                     4 * (d + 4) * heads * t, 4), 0, 2, 1, 3)
+    y = lib.ggml_set_rows(ctx, C, src, I)
+    G.gf = lib.ggml_new_graph_custom(ctx, G.graph_size, False)
+    lib.ggml_build_forward_expand(G.gf, y)
+    G.allocate(gpu.buft)
+    x = RNG.standard_normal((n, t, heads, d + 4 * skip)).astype(np.float32) * 3
+    rows = np.stack([RNG.permutation(span)[:t] for _ in range(n)])
+    want = RNG.standard_normal((n, heads, span, d)).astype(np.float16)
+    G.set(C, want)
+    G.set(X, x)
+    G.set(I, rows.astype(np.int64 if i64 else np.int32))
+    assert G.compute(gpu.backend) == 0
+    part = x[..., 1:1 + d] if skip else x
+    for s in range(n):
+        want[s][:, rows[s]] = part[s].transpose(1, 0, 2).astype(np.float16)
+    assert np.array_equal(G.get(C, np.uint16).reshape(-1), want.view(np.uint16).reshape(-1))
+    G.free()
+
+
+@pytest.mark.parametrize("heads,kv_heads,t", [(16, 8, 256), (16, 8, 255), (6, 2, 1000), (4, 4, 1024)])
+def test_norm_rope_rows(ggml, gpu, heads, kv_heads, t):
+    """RMS_NORM, weight and RoPE of the query and key rows: four heads of a
+    position a wave (many rows, heads in fours) or one, the same bits as the
+    three ops apart"""
+    print(f"norm rope {heads}/{kv_heads} x {t}", flush=True)
+    d, outs = 128, []
+    x = RNG.standard_normal((t, (heads + kv_heads) * d)).astype(np.float32)
+    w = RNG.uniform(0.5, 1.5, (2, d)).astype(np.float32)
+    for fused in (True, False):
+        G = ggml.Graph()
+        lib, ctx = G.lib, G.ctx
+        X = [G.new(ggml.F32, d, h, t) for h in (heads, kv_heads)]
+        W = [G.new(ggml.F32, d, weight=True) for _ in range(2)]
+        P = G.new(ggml.I32, t)
+        keep, out = [], []
+        for a, b in zip(X, W):
+            a = lib.ggml_rms_norm(ctx, a, 1e-6)
+            b = lib.ggml_mul(ctx, a, b)
+            keep += [a, b]
+            out.append(lib.ggml_rope_ext(ctx, b, P, None, d, ggml.GGML_ROPE_TYPE_NEOX, 4096, 1e6, 1.0, 0.0, 1.0, 32.0, 1.0))
+        G.build(*(out if fused else keep + out))  # intermediate results that are outputs are not folded
+        G.allocate(gpu.buft)
+        G.set(X[0], x[:, :heads * d]), G.set(X[1], x[:, heads * d:])
+        G.set(W[0], w[0]), G.set(W[1], w[1])
+        G.set(P, (np.arange(t) * 3 + 5).astype(np.int32))
+        assert G.compute(gpu.backend) == 0
+        outs.append(np.concatenate([G.get(o).reshape(-1) for o in out]))
+        G.free()
+    assert np.array_equal(outs[0].view(np.uint32), outs[1].view(np.uint32))
