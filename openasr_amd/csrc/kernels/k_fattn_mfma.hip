@@ -59,21 +59,10 @@ __device__ __forceinline__ fm_h8 fm_load8(const _Float16 * p) { return *(const f
 // entry's page); 3 4-byte rows -- four word loads the same way; 2 other
 // rows -- eight 2-byte loads, indexes clamped below n_kv. fm_mask_fix:
 // positions at or past n_kv become -inf.
-// MM 4: an f32 mask, rounded to f16 (what its CPY to an f16 mask would hold).
 template <int MM>
 __device__ __forceinline__ fm_u4 fm_mask_load(const uint16_t * row, int pos, int n_kv) {
     if constexpr (MM == 0) {
         return fm_u4{0, 0, 0, 0};
-    } else if constexpr (MM == 4) {
-        const float * f = (const float *) row;
-        float v[8];
-#pragma unroll
-        for (int j = 0; j < 8; j++) v[j] = f[min(pos + j, n_kv - 1)];
-        fm_u4 r;
-#pragma unroll
-        for (int j = 0; j < 4; j++)
-            r[j] = (uint32_t) float_to_half_bits(v[2 * j]) | ((uint32_t) float_to_half_bits(v[2 * j + 1]) << 16);
-        return r;
     } else if constexpr (MM == 1) {
         return *(const fm_u4 *) (row + min(pos, (n_kv - 1) & ~7));
     } else if constexpr (MM == 3) {
@@ -136,8 +125,9 @@ __device__ __forceinline__ void fm_merge(float & M, float & L, float m, float l,
 //
 // KV32: K and V are f32 (the encoders' head views of their projections),
 // staged rounded to f16 -- what a copy to f16 tensors ahead of the launch
-// would hold. With MM 4 the three conversion launches of an encoder layer go
-// (a 30 s encode: 11.8 us a layer).
+// would hold: that launch (6.8 us a layer of a 30 s encode) goes, the
+// attention stays at 20 us. Reading an f32 mask here as well, in place of its
+// 5 us cast, measured 27.5 us: its rows on 4 bytes take a load an entry.
 //
 // MG: the workgroup takes every split of its rows in turn and merges
 // their states in registers (fm_merge, in split order, what the combine
@@ -617,13 +607,12 @@ void launch_fattn_mfma(const fattn_args & a, void * scratch, float * out, hipStr
     };
     using d128 = std::integral_constant<int, 128>;
     using d64 = std::integral_constant<int, 64>;
-    if (a.mfma_kv32 || a.mfma_mask32) {
-        if (!fattn_mfma_reads_f32(a) || !a.mfma_kv32) {
+    if (a.mfma_kv32) {
+        if (!fattn_mfma_reads_f32(a)) {
             note_hip_error(hipErrorInvalidValue);
             return;
         }
-        if (a.mfma_mask32) go(k_fattn_mfma<64, 4, false, true>);
-        else if (mm == 0) go(k_fattn_mfma<64, 0, false, true>);
+        if (mm == 0) go(k_fattn_mfma<64, 0, false, true>);
         else if (mm == 1) go(k_fattn_mfma<64, 1, false, true>);
         else if (mm == 3) go(k_fattn_mfma<64, 3, false, true>);
         else go(k_fattn_mfma<64, 2, false, true>);

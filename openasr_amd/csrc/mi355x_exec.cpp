@@ -515,8 +515,6 @@ struct planner {
     bool plan_fattn(int i, const ggml_tensor * t);
     bool make_fattn(const ggml_tensor * t, fattn_args & a);
     bool fattn_kv32(const ggml_tensor * t, const fattn_args & a) const;
-    bool mask32_ok(int i, const ggml_tensor * c);
-    std::unordered_set<const ggml_tensor *> mask32;  // f16 masks not launched: their attention reads the f32 one
     void fattn_quant_out(int i, const ggml_tensor * t, fattn_args & a, const ggml_tensor *& view);
     bool plan_attn_step(int i, const ggml_tensor * t);
 };
@@ -1598,27 +1596,6 @@ bool planner::fattn_kv32(const ggml_tensor * t, const fattn_args & a) const {
            aligned16(a.k) && aligned16(a.v);
 }
 
-// c, planned at node i, is the CPY of an f32 mask that only a matrix-core
-// attention reads, which then reads the f32 mask itself and c is not launched:
-// nothing up to and with that attention writes the f32 mask's bytes
-bool planner::mask32_ok(int i, const ggml_tensor * c) {
-    const ggml_tensor * m = c->src[0];
-    if (c->type != GGML_TYPE_F16 || m->type != GGML_TYPE_F32 || (c->flags & GGML_TENSOR_FLAG_OUTPUT) ||
-        !is_contiguous(c) || !is_contiguous(m) || (c->src[1] && c->src[1] != c) || bypass.count(root_of(m)) || deferred.count(root_of(m)))
-        return false;
-    for (int d = 0; d < 4; d++)
-        if (c->ne[d] != m->ne[d]) return false;
-    const ggml_tensor * t = sole_consumer(c, i + 1);
-    fattn_args a;
-    if (!t || t->op != GGML_OP_FLASH_ATTN_EXT || t->src[3] != c || t->src[0] == c || !supports_op(be->dev, t)) return false;
-    if (no_fold.count(c) || !make_fattn(t, a) || !fattn_kv32(t, a)) return false;
-    const span sm = span_of(m);
-    for (int j = i + 1; j <= index.at(t); j++)
-        if (!is_view_op(cg->nodes[j]->op) && overlap(span_of(cg->nodes[j]), sm)) return false;
-    fold_reads.push_back({c, sm, i, index.at(t)});  // nor a launch moved there (validate)
-    return true;
-}
-
 bool planner::plan_fattn(int i, const ggml_tensor * t) {
     fattn_args a;
     if (!make_fattn(t, a)) return false;
@@ -1635,13 +1612,6 @@ bool planner::plan_fattn(int i, const ggml_tensor * t) {
     gen_need = std::max(gen_need, part + kbytes + vbytes);
     const tview kv = make_view(k), vv = make_view(v);
     a.mfma_kv32 = fattn_kv32(t, a);
-    if (mask32.count(t->src[3])) {
-        // the f32 mask in the place of its CPY (find_mask32's conditions)
-        const ggml_tensor * m = t->src[3]->src[0];
-        a.mfma_mask32 = true;
-        a.mask = (const char *) m->data;
-        a.m_nb1 = m->nb[1], a.m_nb2 = m->nb[2], a.m_nb3 = m->nb[3];
-    }
     backend_state * b = be;
     const int ncu = n_cu;
     float * out = (float *) t->data;
@@ -2108,11 +2078,6 @@ bool planner::plan() {
                 if (naive_jobs.count(t)) {
                     if (!plan_naive(i, t)) return false;
                     continue;
-                }
-                if (t->op == GGML_OP_CPY && mask32_ok(i, t)) {
-                    mask32.insert(t);
-                    deferred[t] = t;
-                    break;
                 }
                 const ggml_tensor * dst = t;
                 const tview dv = make_view(dst), av = view_of(t->src[0]);

@@ -222,7 +222,6 @@ struct fattn_args {
     int mfma_split;  // KV splits of the matrix-core form (partials + combine when > 1)
     bool mfma_merge;  // its splits merged in the workgroup instead
     bool mfma_kv32;   // K and V are f32 (16-byte aligned rows), rounded to f16 as they are staged
-    bool mfma_mask32;  // the mask is f32, rounded to f16 as it is read
     // one query at the default precision: the workgroup form (k_fattn_dec.hip,
     // float tolerance); its KV splits (0: not used; > 1: partials + combine)
     int dec;
@@ -231,7 +230,7 @@ struct fattn_args {
 bool fattn_mfma_supported(const fattn_args & a);
 void fattn_mfma_plan(fattn_args & a, int n_cu);
 size_t fattn_mfma_scratch_bytes(const fattn_args & a);
-// whether the planned matrix-core form reads f32 K and V / an f32 mask itself
+// whether the planned matrix-core form reads f32 K and V itself
 bool fattn_mfma_reads_f32(const fattn_args & a);
 void launch_fattn_mfma(const fattn_args & a, void * scratch, float * out, hipStream_t s);
 struct attn_step_args;
