@@ -28,9 +28,13 @@
 // step is multiplied, then dequantized into the other of two LDS buffers
 // (16-byte pieces XOR-swizzled by row: conflict-free fragment reads, 64 KB
 // of LDS a workgroup); one barrier a
-// step (174 VGPRs + 88 AGPRs: one workgroup a CU; held to two a CU, 256
-// registers a lane, the compiler fits without spills but the GEMM measured
-// 1-5 % slower). Wave (wr, wc) multiplies the 64 x 64 quarter (wr: rows, wc:
+// step. The step's order is given to the compiler (sched_group_barrier): after
+// every MFMA a few vector instructions of the next step's dequantization, so
+// that a wave's matrix and vector work overlap, where they ran one after the
+// other (Q4_K's scale unpacking was a branch that kept them in separate
+// blocks). 214-229 VGPRs, two workgroups a CU (174 + 88 AGPRs and one before);
+// the products above 175 -> 168, 75 -> 67 and 52 -> 51 us. A step still takes a
+// CU about twice its MFMAs' time. Wave (wr, wc) multiplies the 64 x 64 quarter (wr: rows, wc:
 // columns) as 4 x 4 blocks of 16 x 16: the activations are the MFMA A
 // operand (lane l: column l % 16, k 8 (l / 16) .. + 7), the weights the B
 // operand, so lane l ends with weight row l % 16 of four consecutive
@@ -65,6 +69,9 @@ __device__ __forceinline__ uint4 * hq_slot(uint16_t (*a)[kHRow], int row, int pi
 constexpr int kHThreads = 256;
 constexpr int kHXcds = 8;
 constexpr int kHBand = 4;  // column blocks the tile order takes side by side
+
+// instruction classes of __builtin_amdgcn_sched_group_barrier
+constexpr int kSchedValu = 0x2, kSchedMfma = 0x8, kSchedDsRead = 0x100, kSchedDsWrite = 0x200;
 
 typedef _Float16 hh2 __attribute__((ext_vector_type(2)));
 typedef _Float16 hh8 __attribute__((ext_vector_type(8)));
@@ -173,15 +180,16 @@ __device__ __forceinline__ void hq_store(const hq_regs & r, int64_t k0, uint16_t
         // get_scale_min_k4 of the header's 12 scale bytes
         const int c = (int) ((k0 % 256) / 64);
         const uint32_t s0 = r.hdr.y, s1 = r.hdr.z, s2 = r.hdr.w;
+        // (sub-blocks 4 .. 7 keep four bits in the third word and two above the
+        // lower ones' six: selects and masks, uniform over the step, no branch
+        // -- a branch here keeps the step's matrix and vector work apart)
+        const bool upper = c >= 2;
+        const uint32_t lowmask = upper ? 15u : 63u, topmask = upper ? 3u : 0u;
+        const uint32_t bsc = upper ? s2 : s0, bmn = upper ? s2 >> 4 : s1;
         auto scale_min = [&](int j, float & sc, float & mn) {
-            if (j < 4) {
-                sc = (float) ((s0 >> (8 * j)) & 63);
-                mn = (float) ((s1 >> (8 * j)) & 63);
-            } else {
-                const int q = j - 4;
-                sc = (float) (((s2 >> (8 * q)) & 0xF) | (((s0 >> (8 * q + 6)) & 3) << 4));
-                mn = (float) (((s2 >> (8 * q + 4)) & 0xF) | (((s1 >> (8 * q + 6)) & 3) << 4));
-            }
+            const int sh = 8 * (j & 3);
+            sc = (float) (((bsc >> sh) & lowmask) | (((s0 >> (sh + 6)) & topmask) << 4));
+            mn = (float) (((bmn >> sh) & lowmask) | (((s1 >> (sh + 6)) & topmask) << 4));
         };
         const float d = half_bits_to_float((uint16_t) (r.hdr.x & 0xFFFF));
         const float dmin = half_bits_to_float((uint16_t) (r.hdr.x >> 16));
@@ -301,6 +309,19 @@ __global__ __launch_bounds__(kHThreads) void k_mmq_f16(mmqh_args a) {
                                                                         0, 0);
         }
     };
+    // a step's order: the first fragments' reads, then a few vector
+    // instructions (the next step's dequantization) after every MFMA, with the
+    // second half's reads early and the staging stores late
+    auto interleave = [&]() __attribute__((always_inline)) {
+        __builtin_amdgcn_sched_group_barrier(kSchedDsRead, 8, 0);
+#pragma unroll
+        for (int i = 0; i < 32; i++) {
+            __builtin_amdgcn_sched_group_barrier(kSchedMfma, 1, 0);
+            __builtin_amdgcn_sched_group_barrier(kSchedValu, 4, 0);
+            if (i < 8) __builtin_amdgcn_sched_group_barrier(kSchedDsRead, 1, 0);
+            if (i >= 24) __builtin_amdgcn_sched_group_barrier(kSchedDsWrite, 1, 0);
+        }
+    };
     // step s (set and buffer s % 2): multiply buffer s % 2, store step s + 1
     // into the other buffer -- last read in step s - 1, before the barrier
     // that ended it -- and reload that set with step s + 3
@@ -310,10 +331,12 @@ __global__ __launch_bounds__(kHThreads) void k_mmq_f16(mmqh_args a) {
         compute(0);
         hq_store<WT>(rb, kstep(s + 1), s_w[1], s_x[1]);
         hq_load<WT>(a, wrow, n0, kstep(s + 3), rb);
+        interleave();
         __syncthreads();
         compute(1);
         hq_store<WT>(ra, kstep(s + 2), s_w[0], s_x[0]);
         hq_load<WT>(a, wrow, n0, kstep(s + 4), ra);
+        interleave();
         __syncthreads();
     }
     if constexpr (SWI) {
