@@ -227,6 +227,52 @@ __global__ __launch_bounds__(256) void k_norm(tview d, tview a, int mode, float 
     }
 }
 
+// Rows of 513 to 1024 elements (a multiple of four, 16-byte rows, 1-D weight
+// and bias vectors) that k_norm_rows does not take: a workgroup a row, four
+// elements a thread in one 16-byte load each of row, weight and bias, the f64
+// sums of the four waves added through LDS. Latency bound: in k_norm one wave
+// walks such a row with up to 16 four-byte loads behind exec masks and holds
+// the whole row's sums (390 rows of 896: 6.6 us there, 5.1 us here).
+__global__ __launch_bounds__(256) void k_norm_row4(tview d, tview a, int mode, float eps, const float * __restrict__ wr,
+                                                   const float * __restrict__ br) {
+    __shared__ double s_sum[2][4];
+    const int64_t row = blockIdx.x;
+    const int64_t i1 = row % a.ne[1], i2 = (row / a.ne[1]) % a.ne[2], i3 = row / (a.ne[1] * a.ne[2]);
+    const float * x = (const float *) (a.data + i1 * a.nb[1] + i2 * a.nb[2] + i3 * a.nb[3]);
+    float * y = (float *) (d.data + i1 * d.nb[1] + i2 * d.nb[2] + i3 * d.nb[3]);
+    const int n = (int) a.ne[0], i = 4 * (int) threadIdx.x, wave = (int) threadIdx.x >> 6;
+    const bool ok = i < n;  // past the row: its first elements again, not summed or stored
+    const int at = ok ? i : 0;
+    const float4 one = make_float4(1.0f, 1.0f, 1.0f, 1.0f), zero = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    const float4 x4 = *(const float4 *) (x + at);
+    const float4 w4 = wr ? *(const float4 *) (wr + at) : one, b4 = br ? *(const float4 *) (br + at) : zero;
+    const float xv[4] = {x4.x, x4.y, x4.z, x4.w}, wv[4] = {w4.x, w4.y, w4.z, w4.w}, bv[4] = {b4.x, b4.y, b4.z, b4.w};
+    auto row_sum = [&](double v, int k) {
+        const double w = wave_sum_d(ok ? v : 0.0);
+        if ((threadIdx.x & 63) == 0) s_sum[k][wave] = w;
+        __syncthreads();
+        return s_sum[k][0] + s_sum[k][1] + s_sum[k][2] + s_sum[k][3];
+    };
+    float mean = 0.0f;
+    if (mode == 1) mean = (float) (row_sum((double) xv[0] + (double) xv[1] + (double) xv[2] + (double) xv[3], 0) / (double) n);
+    double s2 = 0.0;
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+        const float v = xv[k] - mean;
+        s2 += (double) (v * v);
+    }
+    const float var = (float) (row_sum(s2, 1) / (double) n);
+    const float scale = 1.0f / sqrtf(var + eps);
+    float o[4];
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+        o[k] = (xv[k] - mean) * scale;
+        if (wr) o[k] *= wv[k];
+        if (br) o[k] += bv[k];
+    }
+    if (ok) *(float4 *) (y + i) = make_float4(o[0], o[1], o[2], o[3]);
+}
+
 // Rows whose width is a multiple of 256 with contiguous elements and 1-D
 // weight / bias vectors: one workgroup per row, its W waves take the row's
 // 256-element chunks round-robin, lane l holding elements 256c + 4l .. +3
@@ -330,11 +376,8 @@ void launch_spin_us(double us, int wall_clock_khz, hipStream_t s) {
     hipLaunchKernelGGL(k_spin, dim3(1), dim3(64), 0, s, ticks);
 }
 
-bool norm_rows_supported(const tview & d, const tview & a, const tview * w, const tview * b) {
-    const int64_t n = a.ne[0];
-    if (n % 256 != 0 || n / 256 > 16) return false;
-    const int c = (int) (n / 256);
-    if (c != 1 && c != 2 && c != 4 && c != 6 && c != 8 && c != 12 && c != 16) return false;
+// 16-byte loads of the rows and of 1-D weight and bias vectors
+static bool norm_aligned(const tview & d, const tview & a, const tview * w, const tview * b) {
     if (a.nb[0] != 4 || d.nb[0] != 4) return false;
     if ((((uintptr_t) a.data) | ((uintptr_t) d.data) | a.nb[1] | a.nb[2] | a.nb[3] | d.nb[1] | d.nb[2] | d.nb[3]) % 16)
         return false;
@@ -343,6 +386,14 @@ bool norm_rows_supported(const tview & d, const tview & a, const tview * w, cons
         if (v->ne[1] != 1 || v->ne[2] != 1 || v->ne[3] != 1 || v->nb[0] != 4 || ((uintptr_t) v->data) % 16) return false;
     }
     return true;
+}
+
+bool norm_rows_supported(const tview & d, const tview & a, const tview * w, const tview * b) {
+    const int64_t n = a.ne[0];
+    if (n % 256 != 0 || n / 256 > 16) return false;
+    const int c = (int) (n / 256);
+    if (c != 1 && c != 2 && c != 4 && c != 6 && c != 8 && c != 12 && c != 16) return false;
+    return norm_aligned(d, a, w, b);
 }
 
 void launch_norm(const tview & d, const tview & a, int mode, float eps, const tview * w, const tview * b,
@@ -364,6 +415,11 @@ void launch_norm(const tview & d, const tview & a, int mode, float eps, const tv
             case 12: hipLaunchKernelGGL((k_norm_rows<12, 4>), g1, dim3(256), 0, s, d, a, mode, eps, wp, bp, qt, ab); return;
             default: hipLaunchKernelGGL((k_norm_rows<16, 4>), g1, dim3(256), 0, s, d, a, mode, eps, wp, bp, qt, ab); return;
         }
+    }
+    if (a.ne[0] > 512 && a.ne[0] <= 1024 && a.ne[0] % 4 == 0 && norm_aligned(d, a, w, b)) {
+        hipLaunchKernelGGL(k_norm_row4, dim3((unsigned) rows), dim3(256), 0, s, d, a, mode, eps,
+                           w ? (const float *) w->data : nullptr, b ? (const float *) b->data : nullptr);
+        return;
     }
     const int per = (int) ((a.ne[0] + 63) / 64);
     tview none{};

@@ -309,3 +309,36 @@ def test_norm_rope_rows(ggml, gpu, heads, kv_heads, t):
         outs.append(np.concatenate([G.get(o).reshape(-1) for o in out]))
         G.free()
     assert np.array_equal(outs[0].view(np.uint32), outs[1].view(np.uint32))
+
+
+@pytest.mark.parametrize("n", [512, 516, 640, 896, 1020, 1028])
+@pytest.mark.parametrize("rows", [1, 390])
+@pytest.mark.parametrize("layer", [False, True])
+def test_norm_row_widths(ggml, gpu, n, rows, layer):
+    """RMS_NORM and NORM with weight and bias at the edges of the
+    workgroup-a-row form (513 to 1024 elements, a multiple of four)"""
+    f = np.float32
+    x = (RNG.standard_normal((rows, n)) * 2 + 0.7).astype(f)
+    w, b = RNG.uniform(0.5, 1.5, n).astype(f), RNG.standard_normal(n).astype(f)
+    G = ggml.Graph()
+    lib, ctx = G.lib, G.ctx
+    X, W, B = G.new(ggml.F32, n, rows), G.new(ggml.F32, n, weight=True), G.new(ggml.F32, n, weight=True)
+    y = lib.ggml_norm(ctx, X, 1e-5) if layer else lib.ggml_rms_norm(ctx, X, 1e-5)
+    y = lib.ggml_mul(ctx, y, W)
+    if layer:
+        y = lib.ggml_add(ctx, y, B)
+    G.build(y)
+    G.allocate(gpu.buft)
+    G.set(X, x), G.set(W, w), G.set(B, b)
+    assert G.compute(gpu.backend) == 0
+    mean = (x.astype(np.float64).sum(1, keepdims=True) / n).astype(f) if layer else f(0)
+    v = x - mean
+    var = ((v * v).astype(np.float64).sum(1, keepdims=True) / n).astype(f)
+    want = v * (f(1) / np.sqrt(var + f(1e-5))) * w
+    if layer:
+        want = want + b
+    got = G.get(y).reshape(rows, n)
+    # the same f32 steps around f64 sums: a row moves only where its sum lies
+    # on an f32 rounding boundary, and then by one step of its mean or scale
+    assert (got != want).mean() <= 0.01 and np.abs(got - want).max() <= 4 * 2.0 ** -23 * np.abs(want).max()
+    G.free()
