@@ -318,7 +318,7 @@ __global__ __launch_bounds__(64 * RW * KW) void k_mmq(mmq_args a) {
             float v = (float) acc[grp][i];
             if (n < a.N) {
                 if (a.epi.bias) v = v + a.epi.bias[row];
-                if (a.epi.res) v = v + *(const float *) ((const char *) a.epi.res + (int64_t) n * a.dst_nb1 + row * 4);
+                if (a.epi.res) v = v + a.epi.res[(int64_t) n * a.M + row];
             }
             o[grp * 4 + i] = v;
         }

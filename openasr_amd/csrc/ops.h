@@ -124,7 +124,9 @@ struct gemm_float_epi {
     bool gelu_erf = false;
     const float * bias_col = nullptr;
     int64_t perm_rows = 0;
-    bool f16_out = false;  // launch_mmq: the result rounded to f16 (dst_nb1 in bytes of it)
+    // launch_mmq: the result rounded to f16 (dst_nb1 in bytes of it; the
+    // residual's columns stay f32, M apart)
+    bool f16_out = false;
 };
 constexpr int kGemmFloatMaxSubs = 2;
 struct gemm_float_args {

@@ -342,3 +342,54 @@ def test_norm_row_widths(ggml, gpu, n, rows, layer):
     # on an f32 rounding boundary, and then by one step of its mean or scale
     assert (got != want).mean() <= 0.01 and np.abs(got - want).max() <= 4 * 2.0 ** -23 * np.abs(want).max()
     G.free()
+
+
+def gelu_erf_f32(z):
+    from math import erf
+    a = z * np.float32(0.70710678118654752440)
+    e = np.array([erf(float(v)) for v in a.reshape(-1)], np.float32).reshape(z.shape)
+    return np.float32(0.5) * z * (np.float32(1) + e)
+
+
+@pytest.mark.parametrize("wname,m,k,n", [("q8_0", 64, 352, 97), ("q4_K", 80, 512, 65)])
+@pytest.mark.parametrize("bias,res,gelu", [(False, False, True), (False, True, False), (False, True, True),
+                                           (True, True, False), (True, True, True)])
+def test_product_epilogues_into_f16_tensors(ggml, gpu, ref, wname, m, k, n, bias, res, gelu):
+    """a product with a bias, a residual and a GELU_ERF copied into an f16
+    tensor: the f16 of the f32 steps (the residual's rows are f32 rows, whatever
+    the result's are)"""
+    print(f"f16 epilogue {wname} {m} x {k} x {n} bias {bias} res {res} gelu {gelu}", flush=True)
+    wt = ggml.Q8_0 if wname == "q8_0" else ggml.Q4_K
+    G = ggml.Graph()
+    lib, ctx = G.lib, G.ctx
+    X, R = G.new(ggml.F32, k, n), G.new(ggml.F32, m, n)
+    W, B, C = G.new(wt, k, m, weight=True), G.new(ggml.F32, m, weight=True), G.new(ggml.F16, m, n, weight=True)
+    y = lib.ggml_mul_mat(ctx, W, X)
+    lib.ggml_mul_mat_set_prec(y, ggml.GGML_PREC_F32)
+    if bias:
+        y = lib.ggml_add(ctx, y, B)
+    if res:
+        y = lib.ggml_add(ctx, y, R)
+    if gelu:
+        y = lib.ggml_gelu_erf(ctx, y)
+    G.build(lib.ggml_cpy(ctx, y, C))
+    G.allocate(gpu.buft)
+    x, r = RNG.standard_normal((n, k)).astype(np.float32), RNG.standard_normal((n, m)).astype(np.float32)
+    b = RNG.standard_normal(m).astype(np.float32)
+    wq = ggml.quantize(wt, ggml.synth_normal(5, m, m * k, 0.0, 0.02).reshape(m, k))
+    G.set(W, wq), G.set(B, b)
+    want = ref.mul_mat(wt, wq, m, k, x)
+    if bias:
+        want = want + b
+    if res:
+        want = want + r
+    if gelu:
+        want = gelu_erf_f32(want)
+    for _ in range(3):
+        G.set(X, x)
+        if res:
+            G.set(R, r)
+        assert G.compute(gpu.backend) == 0
+        # an f32 step apart once in ~2^27 values, and an f16 once in ~2^40
+        assert np.array_equal(G.get(C, np.uint16).reshape(n, m), want.astype(np.float16).view(np.uint16))
+    G.free()
