@@ -395,6 +395,9 @@ struct planner {
         for (const ggml_tensor * w : writes) {
             const span sp = span_of(w);
             if (sp.lo < sp.hi) s.writes.push_back({sp.lo, sp.hi});
+            // the act region no longer holds what these bytes quantize to (a
+            // step that quantizes its own result sets act_src after itself)
+            if (act_src && overlap(sp, span_of(act_src))) act_src = nullptr;
         }
         if (plan_trace()) {
             std::fprintf(stderr, "mi355x plan: step %zu at node %d %s", steps.size(), cur, label);
@@ -2151,11 +2154,6 @@ bool planner::plan() {
             default:
                 return fail(t, "no launcher");
         }
-        // a node other than MUL_MAT may overwrite memory the act region was
-        // quantized from only through a view; be conservative for writers
-        // a write through a view may change the columns the act region holds
-        if ((t->op == GGML_OP_SET_ROWS || t->op == GGML_OP_CPY) && act_src && overlap(span_of(t), span_of(act_src)))
-            act_src = nullptr;
     }
     return true;
 }

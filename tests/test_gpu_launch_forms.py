@@ -393,3 +393,47 @@ def test_product_epilogues_into_f16_tensors(ggml, gpu, ref, wname, m, k, n, bias
         # an f32 step apart once in ~2^27 values, and an f16 once in ~2^40
         assert np.array_equal(G.get(C, np.uint16).reshape(n, m), want.astype(np.float16).view(np.uint16))
     G.free()
+
+
+# 80 rows: two launches over one quantization of the columns
+@pytest.mark.parametrize("m", [80])
+@pytest.mark.parametrize("how", ["pair", "rows", "copy"])
+@pytest.mark.parametrize("wname", ["q8_0", "q4_K"])
+def test_columns_written_between_products(ggml, gpu, ref, wname, m, how):
+    """product, a write over some of its columns (the second of two SET_ROWS of
+    the same rows, one SET_ROWS, or a copy), product: the second one sees the
+    written columns"""
+    print(f"columns written between products {wname} {m} {how}", flush=True)
+    k, n, rows = 512, 97, 5
+    wt = ggml.Q8_0 if wname == "q8_0" else ggml.Q4_K
+    G = ggml.Graph()
+    lib, ctx = G.lib, G.ctx
+    X, A = G.new(ggml.F32, k, n, weight=True), G.new(ggml.F32, k, n, weight=True)
+    W = [G.new(wt, k, m, weight=True) for _ in range(2)]
+    V, I = G.new(ggml.F32, k, rows), G.new(ggml.I32, rows)
+    G.gf = lib.ggml_new_graph_custom(ctx, G.graph_size, False)
+    Y = [lib.ggml_mul_mat(ctx, w, X) for w in W]
+    writes = {"pair": lambda: [lib.ggml_set_rows(ctx, A, V, I), lib.ggml_set_rows(ctx, X, V, I)],
+              "rows": lambda: [lib.ggml_set_rows(ctx, X, V, I)],
+              "copy": lambda: [lib.ggml_cpy(ctx, V, lib.ggml_view_2d(ctx, X, k, rows, 4 * k, 4 * k * 30))]}[how]()
+    for t in (Y[0], *writes, Y[1]):
+        lib.ggml_build_forward_expand(G.gf, t)
+    for y in Y:
+        lib.ggml_set_output(y)
+    G.allocate(gpu.buft)
+    x, v = RNG.standard_normal((n, k)).astype(np.float32), RNG.standard_normal((rows, k)).astype(np.float32)
+    at = np.arange(30, 30 + rows) if how == "copy" else np.array([96, 0, 17, 64, 3])
+    wq = [ggml.quantize(wt, ggml.synth_normal(6, i, m * k, 0.0, 0.02).reshape(m, k)) for i in range(2)]
+    for t, q in zip(W, wq):
+        G.set(t, q)
+    after = x.copy()
+    after[at] = v
+    want = [ref.mul_mat(wt, wq[0], m, k, x), ref.mul_mat(wt, wq[1], m, k, after)]
+    for _ in range(3):
+        G.set(X, x), G.set(V, v)
+        if how != "copy":
+            G.set(I, at.astype(np.int32))
+        assert G.compute(gpu.backend) == 0
+        for y, z in zip(Y, want):
+            assert np.abs(G.get(y).reshape(n, m) - z).max() <= 2.0 ** -22 * np.abs(z).max()
+    G.free()
