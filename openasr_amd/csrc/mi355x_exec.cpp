@@ -475,8 +475,8 @@ struct planner {
         hi = lo + (uintptr_t) last;
     }
 
-    // no node between positions i and j (inclusive) that may run writes into
-    // the bytes of view v
+    // no node from position i + 1 to j that may run writes into the bytes of
+    // view v
     bool untouched_until(const tview & v, int i, int j) const {
         uintptr_t lo, hi;
         view_span(v, 4, lo, hi);
@@ -820,6 +820,10 @@ bool planner::plan_mul_mat(int i, const ggml_tensor * t) {
             h = h2;
             return true;
         };
+        // a later product u of the same columns may run in this launch: nothing
+        // from here up to it writes them (hoist_ok sees what a launch reads,
+        // and a launch over quantized columns does not read x itself)
+        auto columns_last = [&](const ggml_tensor * u) { return untouched_until(xv, i - 1, index.at(u) - 1); };
         // the default precision (the graph's contract, op_params[0]) with
         // enough tiles and 16-byte weight rows: the f16 matrix-core form
         // (k_mmq_f16.hip, float tolerance)
@@ -840,7 +844,7 @@ bool planner::plan_mul_mat(int i, const ggml_tensor * t) {
                       u->src[0]->ne[0] == K && u->src[0]->ne[1] == M && u->src[0]->nb[1] == w->nb[1] &&
                       sole_consumer(u, i + 1) == hm && supports_op(be->dev, u) && is_contiguous(hm) &&
                       ready_before(u->src[0], i) && u->op_params[0] == t->op_params[0] &&
-                      (mfma || aligned16(u->src[0]->data));
+                      (mfma || aligned16(u->src[0]->data)) && columns_last(u);
             for (int d = 0; d < 4 && ok; d++) ok = hm->ne[d] == t->ne[d] && u->ne[d] == t->ne[d];
             if (ok && try_fold({silu, u, hm}, hm, {u->src[0]}, nullptr)) {
                 W2 = (const char *) u->src[0]->data;
@@ -911,7 +915,7 @@ bool planner::plan_mul_mat(int i, const ggml_tensor * t) {
                                      uw->ne[0] == K && uw->ne[2] == 1 && uw->ne[3] == 1 &&
                                      (int64_t) uw->nb[1] == row_bytes && uw->ne[1] % 64 == 0 &&
                                      u->type == GGML_TYPE_F32 && is_contiguous(u) && u->ne[1] == N && u->ne[2] == 1 &&
-                                     u->ne[3] == 1 && ready_before(uw, i);
+                                     u->ne[3] == 1 && ready_before(uw, i) && columns_last(u);
                 if (!sibling) continue;
                 gemm_float_sub sb;
                 sb.a = (const char *) uw->data;

@@ -395,8 +395,9 @@ def test_product_epilogues_into_f16_tensors(ggml, gpu, ref, wname, m, k, n, bias
     G.free()
 
 
-# 80 rows: two launches over one quantization of the columns
-@pytest.mark.parametrize("m", [80])
+# 80 rows: two launches over one quantization of the columns; 64: a second
+# product that could join the first one's launch
+@pytest.mark.parametrize("m", [80, 64])
 @pytest.mark.parametrize("how", ["pair", "rows", "copy"])
 @pytest.mark.parametrize("wname", ["q8_0", "q4_K"])
 def test_columns_written_between_products(ggml, gpu, ref, wname, m, how):
@@ -436,4 +437,36 @@ def test_columns_written_between_products(ggml, gpu, ref, wname, m, how):
         assert G.compute(gpu.backend) == 0
         for y, z in zip(Y, want):
             assert np.abs(G.get(y).reshape(n, m) - z).max() <= 2.0 ** -22 * np.abs(z).max()
+    G.free()
+
+
+def test_columns_written_between_gate_and_up(ggml, gpu, ref):
+    """the same between the two products of a SwiGLU whose matrix is too tall
+    for a launch that quantizes its columns itself"""
+    m, k, n = 8224, 256, 4
+    G = ggml.Graph()
+    lib, ctx = G.lib, G.ctx
+    X = G.new(ggml.F32, k, n, weight=True)
+    W = [G.new(ggml.Q8_0, k, m, weight=True) for _ in range(2)]
+    V, I = G.new(ggml.F32, k, 1), G.new(ggml.I32, 1)
+    G.gf = lib.ggml_new_graph_custom(ctx, G.graph_size, False)
+    gate, up = (lib.ggml_mul_mat(ctx, w, X) for w in W)
+    h = lib.ggml_mul(ctx, lib.ggml_silu(ctx, gate), up)
+    for t in (gate, lib.ggml_set_rows(ctx, X, V, I), h):
+        lib.ggml_build_forward_expand(G.gf, t)
+    lib.ggml_set_output(h)
+    G.allocate(gpu.buft)
+    x, v = RNG.standard_normal((n, k)).astype(np.float32), RNG.standard_normal((1, k)).astype(np.float32)
+    wq = [ggml.quantize(ggml.Q8_0, ggml.synth_normal(6, i, m * k, 0.0, 0.05).reshape(m, k)) for i in range(2)]
+    for t, q in zip(W, wq):
+        G.set(t, q)
+    after = x.copy()
+    after[2] = v[0]
+    a, b = ref.mul_mat(ggml.Q8_0, wq[0], m, k, x), ref.mul_mat(ggml.Q8_0, wq[1], m, k, after)
+    want = a.astype(np.float64) / (1 + np.exp(-a.astype(np.float64))) * b
+    for _ in range(3):
+        G.set(X, x), G.set(V, v), G.set(I, np.array([2], np.int32))
+        assert G.compute(gpu.backend) == 0
+        # f32 steps of the SiLU and the product
+        assert np.abs(G.get(h).reshape(n, m) - want).max() <= 2.0 ** -20 * np.abs(want).max()
     G.free()
