@@ -1430,8 +1430,9 @@ bool planner::plan_norm(int i, const ggml_tensor * t) {
     int qt = quant_consumers(out, i + 1);
     if (qt >= 0 && !(out->flags & GGML_TENSOR_FLAG_OUTPUT) && prologue_view(av) && av.ne[0] == out->ne[0] &&
         (!hw || aligned16(wt->data)) && (!hb || aligned16(bt->data))) {
-        // every consumer a prologue GEMV, and the norm's input still intact
-        // when the last of them runs
+        // every consumer a prologue GEMV, the norm's input still intact when
+        // the last of them runs, and nothing written over the norm's result
+        // (which is not materialised) before that
         bool ok = true;
         int last = i;
         for (int j = i + 1; j < cg->n_nodes && ok; j++) {
@@ -1441,7 +1442,7 @@ bool planner::plan_norm(int i, const ggml_tensor * t) {
                 last = j;
             }
         }
-        if (ok && last > i && untouched_until(av, i, last)) {
+        if (ok && last > i && untouched_until(av, i, last) && untouched_until(dv, index.at(out), last)) {
             gemv_prologue p;
             p.x = (const float *) av.data;
             p.x_nb1 = av.nb[1];

@@ -470,3 +470,44 @@ def test_columns_written_between_gate_and_up(ggml, gpu, ref):
         # f32 steps of the SiLU and the product
         assert np.abs(G.get(h).reshape(n, m) - want).max() <= 2.0 ** -20 * np.abs(want).max()
     G.free()
+
+
+@pytest.mark.parametrize("n", [1, 4, 97])
+def test_norm_result_written_between_products(ggml, gpu, ref, n):
+    """a norm's result, a product, a SET_ROWS over the result, a product: the
+    second one sees the written row (products of few columns normalise for
+    themselves where nothing writes between)"""
+    print(f"norm result written between products {n}", flush=True)
+    k, m, f = 512, 80, np.float32
+    G = ggml.Graph()
+    lib, ctx = G.lib, G.ctx
+    X, V, I = G.new(ggml.F32, k, n), G.new(ggml.F32, k, 1), G.new(ggml.I32, 1)
+    N = G.new(ggml.F32, k, weight=True)
+    W = [G.new(ggml.Q8_0, k, m, weight=True) for _ in range(2)]
+    h = lib.ggml_mul(ctx, lib.ggml_rms_norm(ctx, X, 1e-5), N)
+    Y = [lib.ggml_mul_mat(ctx, w, h) for w in W]
+    G.gf = lib.ggml_new_graph_custom(ctx, G.graph_size, False)
+    for t in (Y[0], lib.ggml_set_rows(ctx, h, V, I), Y[1]):
+        lib.ggml_build_forward_expand(G.gf, t)
+    for y in Y:
+        lib.ggml_set_output(y)
+    G.allocate(gpu.buft)
+    x, v = RNG.standard_normal((n, k)).astype(f), RNG.standard_normal((1, k)).astype(f)
+    w = RNG.uniform(0.5, 1.5, k).astype(f)
+    wq = [ggml.quantize(ggml.Q8_0, ggml.synth_normal(8, i, m * k, 0.0, 0.02).reshape(m, k)) for i in range(2)]
+    for t, q in zip(W, wq):
+        G.set(t, q)
+    G.set(N, w)
+    var = ((x * x).astype(np.float64).sum(1, keepdims=True) / k).astype(f)
+    cols = x * (f(1) / np.sqrt(var + f(1e-5))) * w
+    after = cols.copy()
+    after[n - 1] = v[0]
+    want = [ref.mul_mat(ggml.Q8_0, q, m, k, c) for q, c in zip(wq, (cols, after))]
+    for _ in range(3):
+        G.set(X, x), G.set(V, v), G.set(I, np.array([n - 1], np.int32))
+        assert G.compute(gpu.backend) == 0
+        for y, z in zip(Y, want):
+            # a norm's f32 rounding may move by a step and take an 8-bit
+            # activation over its rounding boundary: a step of one of k terms
+            assert np.abs(G.get(y).reshape(n, m) - z).max() <= 0.02 * np.abs(z).max()
+    G.free()
