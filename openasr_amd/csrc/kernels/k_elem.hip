@@ -634,7 +634,9 @@ void launch_set_rows(const tview & dst, int dtype, const tview & src, const tvie
     }
     const int64_t n = j0.n > j1.n ? j0.n : j1.n;
     if (set_rows_f16_ok(j0) && set_rows_f16_ok(j1)) {
-        hipLaunchKernelGGL(k_set_rows_f16, dim3((unsigned) ((n / 8 + 255) / 256), dst2 ? 2 : 1), dim3(256), 0, s, j0, j1);
+        // (no rows at all: one workgroup that writes nothing)
+        const unsigned blocks = (unsigned) std::max<int64_t>(1, (n / 8 + 255) / 256);
+        hipLaunchKernelGGL(k_set_rows_f16, dim3(blocks, dst2 ? 2 : 1), dim3(256), 0, s, j0, j1);
         return;
     }
     hipLaunchKernelGGL(k_set_rows, dim3(grid_for(n, 256, n_cu), dst2 ? 2 : 1), dim3(256), 0, s, j0, j1);

@@ -511,3 +511,34 @@ def test_norm_result_written_between_products(ggml, gpu, ref, n):
             # activation over its rounding boundary: a step of one of k terms
             assert np.abs(G.get(y).reshape(n, m) - z).max() <= 0.02 * np.abs(z).max()
     G.free()
+
+
+@pytest.mark.parametrize("d", [64, 20])
+@pytest.mark.parametrize("second", [0, 3])
+def test_set_rows_of_no_rows(ggml, gpu, d, second):
+    """SET_ROWS of no rows into an f16 cache, alone or before a graph's other
+    work: nothing happens to the cache"""
+    print(f"set_rows of no rows {d} {second}", flush=True)
+    G = ggml.Graph()
+    lib, ctx = G.lib, G.ctx
+    X, I = G.new(ggml.F32, d, 0), G.new(ggml.I32, 0)
+    Y, J = G.new(ggml.F32, d, 3), G.new(ggml.I32, 3)
+    C = [G.new(ggml.F16, d, 9, weight=True) for _ in range(2)]
+    G.gf = lib.ggml_new_graph_custom(ctx, G.graph_size, False)
+    lib.ggml_build_forward_expand(G.gf, lib.ggml_set_rows(ctx, C[0], X, I))
+    if second:
+        lib.ggml_build_forward_expand(G.gf, lib.ggml_set_rows(ctx, C[1], Y, J))
+    G.allocate(gpu.buft)
+    c, y = RNG.standard_normal((2, 9, d)).astype(np.float16), RNG.standard_normal((3, d)).astype(np.float32)
+    want = c.copy()
+    if second:
+        want[1][[8, 0, 5]] = y.astype(np.float16)
+    for _ in range(3):
+        for i in range(2):
+            G.set(C[i], c[i])
+        if second:
+            G.set(Y, y), G.set(J, np.array([8, 0, 5], np.int32))
+        assert G.compute(gpu.backend) == 0
+        for i in range(2):
+            assert np.array_equal(G.get(C[i], np.uint16).reshape(9, d), want[i].view(np.uint16))
+    G.free()
