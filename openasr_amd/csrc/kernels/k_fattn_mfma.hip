@@ -569,7 +569,7 @@ void fattn_mfma_plan(fattn_args & a, int n_cu) {
 }
 
 size_t fattn_mfma_scratch_bytes(const fattn_args & a) {
-    if (a.mfma_split <= 1) return 0;
+    if (a.mfma_split <= 1 || a.mfma_merge) return 0;
     const int64_t rows = (int64_t) fm_q_blocks(a) * a.hkv * a.n_seq * a.mfma_split * kFmRows;
     return (size_t) rows * (a.d + 2) * sizeof(float);
 }

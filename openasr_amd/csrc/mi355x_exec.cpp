@@ -1594,14 +1594,15 @@ void planner::fattn_quant_out(int i, const ggml_tensor * t, fattn_args & a, cons
 }
 
 // the matrix-core attention t (planned as a) reads its f32 K and V itself:
-// both f32, on 16-byte boundaries, not under its output
+// both f32, allocated on 16-byte boundaries (a graph planned for its scratch
+// before it is allocated counts the copies), not under its output
 bool planner::fattn_kv32(const ggml_tensor * t, const fattn_args & a) const {
     for (int k = 1; k <= 2; k++) {
         tview f;
         if (gqa_fold(t->src[k], f) || overlap(span_of(t), span_of(t->src[k]))) return false;
     }
     return t->src[1]->type == GGML_TYPE_F32 && t->src[2]->type == GGML_TYPE_F32 && fattn_mfma_reads_f32(a) &&
-           aligned16(a.k) && aligned16(a.v);
+           a.k && a.v && aligned16(a.k) && aligned16(a.v);
 }
 
 bool planner::plan_fattn(int i, const ggml_tensor * t) {
@@ -1609,17 +1610,17 @@ bool planner::plan_fattn(int i, const ggml_tensor * t) {
     if (!make_fattn(t, a)) return false;
     const ggml_tensor * view = nullptr;
     if (!a.mfma) fattn_quant_out(i, t, a, view);
-    // f32 K / V: rounded to contiguous f16 copies in scratch after the
-    // partials -- the f16 definition over f16-rounded K / V, the conversion
-    // ggml's GPU backends make as well
+    // f32 K / V the kernel does not read itself: rounded to contiguous f16
+    // copies in scratch after the partials -- the f16 definition over
+    // f16-rounded K / V, the conversion ggml's GPU backends make as well
     const ggml_tensor *k = t->src[1], *v = t->src[2];
+    a.mfma_kv32 = fattn_kv32(t, a);
     const size_t part = (fattn_scratch_bytes(a) + 255) & ~(size_t) 255;
-    const bool k32 = k->type == GGML_TYPE_F32, v32 = v->type == GGML_TYPE_F32;
+    const bool k32 = k->type == GGML_TYPE_F32 && !a.mfma_kv32, v32 = v->type == GGML_TYPE_F32 && !a.mfma_kv32;
     const size_t kbytes = k32 ? ((size_t) ggml_nelements(k) * 2 + 255) & ~(size_t) 255 : 0;
     const size_t vbytes = v32 ? ((size_t) ggml_nelements(v) * 2 + 255) & ~(size_t) 255 : 0;
     gen_need = std::max(gen_need, part + kbytes + vbytes);
     const tview kv = make_view(k), vv = make_view(v);
-    a.mfma_kv32 = fattn_kv32(t, a);
     backend_state * b = be;
     const int ncu = n_cu;
     float * out = (float *) t->data;
@@ -1650,9 +1651,7 @@ bool planner::plan_fattn(int i, const ggml_tensor * t) {
                 nb3 = d.nb[3];
             };
             char * g = gen_base(b);
-            if (la.mfma_kv32) {
-                // read as they are
-            } else if (k32 && v32 && !dense_f32(kv) && !dense_f32(vv)) {
+            if (k32 && v32 && !dense_f32(kv) && !dense_f32(vv)) {
                 // both strided head views: one launch for the two
                 tview dk = f16_dense(kv, g + part), dvw = f16_dense(vv, g + part + kbytes);
                 launch_copy_pair(dk, kv, dvw, vv, GGML_TYPE_F16, GGML_TYPE_F32, s, ncu);

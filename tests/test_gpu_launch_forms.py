@@ -542,3 +542,28 @@ def test_set_rows_of_no_rows(ggml, gpu, d, second):
         for i in range(2):
             assert np.array_equal(G.get(C[i], np.uint16).reshape(9, d), want[i].view(np.uint16))
     G.free()
+
+
+def test_attention_reading_f32_keys_takes_no_copy_scratch(ggml, gpu):
+    """an attention that reads f32 K and V itself runs in fixed scratch which
+    their f16 copies would overflow, with the bits of the arena's"""
+    import ctypes
+    lib = gpu.cdll
+    lib.ggml_backend_mi355x_graph_compute_static.restype = ctypes.c_int
+    lib.ggml_backend_mi355x_graph_compute_static.argtypes = [ctypes.c_void_p, ctypes.c_void_p]
+    lib.ggml_backend_mi355x_static_scratch_bytes.restype = ctypes.c_size_t
+    d, heads, t, kv = 64, 14, 64, 20000
+    G = ggml.Graph()
+    q, k, v = (G.new(ggml.F32, d, heads, n, 1) for n in (t, kv, kv))
+    head = lambda x: G.lib.ggml_permute(G.ctx, x, 0, 2, 1, 3)  # noqa: E731
+    y = G.lib.ggml_flash_attn_ext(G.ctx, head(q), head(k), head(v), None, d ** -0.5, 0.0, 0.0)
+    G.build(y)
+    G.allocate(gpu.buft)
+    for x, n in ((q, t), (k, kv), (v, kv)):
+        G.set(x, RNG.standard_normal((n, heads, d)).astype(np.float32))
+    assert 2 * 2 * d * heads * kv > lib.ggml_backend_mi355x_static_scratch_bytes()
+    assert lib.ggml_backend_mi355x_graph_compute_static(gpu.backend, G.gf) == 0
+    static = G.get(y).copy()
+    assert G.compute(gpu.backend) == 0
+    assert np.isfinite(static).all() and np.array_equal(static, G.get(y))
+    G.free()
