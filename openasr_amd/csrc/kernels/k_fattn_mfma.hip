@@ -542,7 +542,48 @@ static int fm_q_blocks(const fattn_args & a) {
     return (a.n_q + qpw - 1) / qpw;
 }
 
-void fattn_mfma_plan(fattn_args & a, int n_cu) {
+// Whether the splits of a (planned over n_tiles tiles) are merged in the
+// workgroup, by a model of both forms' times in units of T, the 2.0 us that one
+// workgroup alone on a CU takes for a tile (at either head size). F(n) is the
+// time in which the CUs, n workgroups dealt to them, do a tile of each: with
+// heads of 128 two are resident and take 1.39 T, further ones come after them;
+// with heads of 64 two take 1.27 T, three 1.53 T, from four on 0.53 T each.
+// Merged, there are `blocks` workgroups of the whole span; most spans have a
+// masked tail, which these skip: 0.9 of it is counted. Split, there are
+// blocks x splits, each of a part of the span (with heads of 64 they fill the
+// CUs evenly), and the combine and the partials cost 6 T and, with heads of
+// 128, 1/128 T a workgroup. With 64-wide heads the split form reads f32 K and V
+// itself, the merged one copies of them (8 T). So merging is refused where few
+// blocks over a long span would leave CUs idle.
+// Measured, us a call, split / merged (128: 16 query, 8 kv heads; queries, live
+// positions and span, sequences):
+//   128 blocks  256 q 640 of 1024, 2     44 / 38    256 q 2000 of 2048, 2    60 / 80
+//               256 q 1000 of 1024, 2    45 / 49    512 q 8000 of 8192, 1   114 / 253
+//   192 blocks  256 q 1000 of 1024, 3    61 / 49    256 q 3000 of 4096, 3   106 / 113
+//   256 blocks  256 q 1500 of 2048, 4    98 / 68    256 q 8000 of 8192, 4   210 / 256
+//               512 q 3000 of 4096, 2   127 / 113   1024 q 4000 of 4096, 1  123 / 137
+//   320 blocks  256 q 3000 of 4096, 5   162 / 146   256 q 8000 of 8192, 5   261 / 336
+//   504 blocks  2000 q 4000 of 4096, 1  223 / 170
+//   512 blocks  256 q 3000 of 4096, 8   256 / 148
+//   576 blocks                                      288 q 8000 of 8192, 8   459 / 543
+// Heads of 64 over f16 K and V, 6 heads: 256 q 500 of 512, 8 sequences (192
+// blocks) 37 / 29, 1500 of 1500, 4 (576) 101 / 84, 1 (144) 45 / 59; over f32, 14
+// heads: 600 of 600, 8 (1120) 117 / 112, 1300 of 1300, 1 (294) 71 / 84. The rule
+// takes the slower form by up to 8 % at the edges (256 q 1000 of 1024, 2).
+static bool fm_merge_pays(const fattn_args & a, int64_t blocks, int n_tiles, bool kv_f32, int n_cu) {
+    const bool wide = a.d == 128;
+    auto shared = [&](int64_t n) {
+        const double k = (double) ((n + n_cu - 1) / n_cu);
+        return wide ? 1.39 * std::floor(k / 2) + std::fmod(k, 2.0) : std::max(0.53 * k, 0.75 + 0.26 * k);
+    };
+    const int64_t wgs = blocks * a.mfma_split;
+    const double per = (double) ((n_tiles + a.mfma_split - 1) / a.mfma_split);
+    const double merged = 0.9 * n_tiles * shared(blocks) + (kv_f32 && !wide ? 8.0 : 0.0);
+    const double split = (wide ? per * shared(wgs) : 0.53 * n_tiles * (double) blocks / n_cu) + 6.0 + (double) (wgs * a.d) / 16384;
+    return merged <= split;
+}
+
+void fattn_mfma_plan(fattn_args & a, int n_cu, bool kv_f32) {
     // split the span when one sequence's query blocks leave CUs idle: up to
     // two workgroups a CU (their LDS and registers fit twice), at least four
     // tiles a split. Planned from one sequence's shape, so a sequence's rows
@@ -556,16 +597,8 @@ void fattn_mfma_plan(fattn_args & a, int n_cu) {
     // no empty split: every split owns at least one tile
     const int per = (n_tiles + split - 1) / split;
     a.mfma_split = (n_tiles + per - 1) / per;
-    // a batch whose row blocks alone fill the CUs (half of them where the
-    // splits are few) merges the splits in registers: no partials written and
-    // read back, one mask scan a row block. us a call, split and combined
-    // against merged, 256 queries over 3000 of 4096 positions, 16 / 8 heads
-    // of 128: 1 sequence (64 row blocks, 8 splits) 53 / 119, 3 114 / 121,
-    // 4 142 / 124, 8 270 / 159; over 640 of 1024 positions (4 splits): 1
-    // 35 / 40, 2 47 / 40, 8 120 / 51.
-    const int64_t blocks = base * a.n_seq;
-    a.mfma_merge = a.mfma_split > 1 && a.n_kv <= kFmMaxSpan &&
-                        (blocks >= n_cu || (a.mfma_split <= 4 && 2 * blocks >= n_cu));
+    // merged or split, the bits are the same
+    a.mfma_merge = a.mfma_split > 1 && a.n_kv <= kFmMaxSpan && fm_merge_pays(a, base * a.n_seq, n_tiles, kv_f32, n_cu);
 }
 
 size_t fattn_mfma_scratch_bytes(const fattn_args & a) {

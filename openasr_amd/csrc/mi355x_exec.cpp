@@ -1562,7 +1562,7 @@ bool planner::make_fattn(const ggml_tensor * t, fattn_args & a) {
     // more than one query at the default precision (op_params[3], the
     // host's flash-attention precision contract): the matrix-core form
     a.mfma = t->op_params[3] != GGML_PREC_F32 && fattn_mfma_supported(a);
-    if (a.mfma) fattn_mfma_plan(a, n_cu);
+    if (a.mfma) fattn_mfma_plan(a, n_cu, k->type == GGML_TYPE_F32 && v->type == GGML_TYPE_F32);
     // one query at the default precision: one workgroup per (sequence, kv
     // head, KV split), the waves merged in the launch (k_fattn_dec.hip),
     // where that form is the faster one

@@ -230,7 +230,7 @@ struct fattn_args {
 };
 // whether the matrix-core form takes this attention (n_q > 1, D 64 / 128)
 bool fattn_mfma_supported(const fattn_args & a);
-void fattn_mfma_plan(fattn_args & a, int n_cu);
+void fattn_mfma_plan(fattn_args & a, int n_cu, bool kv_f32);
 size_t fattn_mfma_scratch_bytes(const fattn_args & a);
 // whether the planned matrix-core form reads f32 K and V itself
 bool fattn_mfma_reads_f32(const fattn_args & a);

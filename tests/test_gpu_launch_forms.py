@@ -118,9 +118,11 @@ def test_products_into_f16_tensors(ggml, gpu, ref, wname, m, k, n, over_columns)
 
 
 # heads, kv heads, sequences, queries, span, live: split and combined (one
-# sequence), merged in the workgroup (a batch), one split, spans off the tile
+# sequence), merged in the workgroup (a batch), one split, spans off the tile; a
+# sequence of 128 blocks over a long span and one of 266, split alone
 @pytest.mark.parametrize("d,hq,hkv,t,span,live", [
     (128, 16, 8, 256, 512, 481), (128, 16, 8, 119, 1024, 1000), (64, 6, 6, 130, 600, 577), (128, 8, 1, 33, 300, 290),
+    (128, 16, 8, 512, 4096, 3000), (64, 14, 14, 1216, 1216, 1216),
 ])
 @pytest.mark.parametrize("scale", [None, -0.11])
 def test_attention_batched_rows_keep_their_bits(ggml, gpu, d, hq, hkv, t, span, live, scale):
@@ -189,7 +191,7 @@ def test_gelu_erf_against_math_erf(ggml, gpu):
     G.free()
 
 
-@pytest.mark.parametrize("heads,t,n", [(14, 390, 1), (3, 97, 1), (2, 64, 2), (1, 2, 3)])
+@pytest.mark.parametrize("heads,t,n", [(14, 390, 1), (14, 1170, 1), (3, 97, 1), (2, 64, 2), (1, 2, 3)])
 @pytest.mark.parametrize("overwritten", [False, True])
 def test_attention_over_f32_keys_and_mask(ggml, gpu, heads, t, n, overwritten):
     """an encoder's attention over strided f32 K / V head views and a mask cast
