@@ -484,10 +484,18 @@ __global__ __launch_bounds__(kFmThreads) void k_fattn_mfma(fattn_args a, float *
     // out = O / l, ggml's [D, hq, n_q, n_seq] layout
     const int r = 16 * wave + l16, i = q0 + r / g;
     if (i >= a.n_q) return;
-    const float sum = MG ? L : l, inv = sum > 0.0f ? 1.0f / sum : 0.0f;
     float * op = out + (((int64_t) seq * a.n_q + i) * a.hq + kvh * g + r % g) * D;
+    const float inv = l > 0.0f ? 1.0f / l : 0.0f;
 #pragma unroll
-    for (int ct = 0; ct < NT; ct++) *(fm_f4 *) &op[16 * ct + 4 * lg] = (MG ? O[ct] : o[ct]) * inv;
+    for (int ct = 0; ct < NT; ct++) {
+        fm_f4 v = fm_f4{0.f, 0.f, 0.f, 0.f};
+        if constexpr (MG) {
+            if (L > 0.0f) v = O[ct] / L;  // as the combine launch divides
+        } else {
+            v = o[ct] * inv;
+        }
+        *(fm_f4 *) &op[16 * ct + 4 * lg] = v;
+    }
 }
 
 // the splits of a workgroup row merged in split order (fm_merge), then out =
@@ -533,8 +541,7 @@ __global__ __launch_bounds__(kFmThreads) void k_fattn_mfma_combine(fattn_args a,
             acc = acc * wa + oz[k] * wb;
         }
     }
-    const float inv = L > 0.0f ? 1.0f / L : 0.0f;
-    out[(((int64_t) seq * a.n_q + i) * a.hq + head) * D + dim] = acc * inv;
+    out[(((int64_t) seq * a.n_q + i) * a.hq + head) * D + dim] = L > 0.0f ? acc / L : 0.0f;
 }
 
 static int fm_q_blocks(const fattn_args & a) {

@@ -569,3 +569,29 @@ def test_attention_reading_f32_keys_takes_no_copy_scratch(ggml, gpu):
     assert G.compute(gpu.backend) == 0
     assert np.isfinite(static).all() and np.array_equal(static, G.get(y))
     G.free()
+
+
+@pytest.mark.parametrize("d,hq,hkv", [(128, 16, 8), (64, 6, 6)])
+@pytest.mark.parametrize("seqs,live", [(1, 1000), (8, 1000), (8, 741)])
+def test_attention_divides_by_the_row_sum(ggml, gpu, d, hq, hkv, seqs, live):
+    """equal scores over splits, combined or merged: the mean of equal values is
+    the value, exactly, as every sum is a whole number below 2^24 and the result
+    one division"""
+    print(f"attention row sums {d} x {seqs} live {live}", flush=True)
+    t, span = 256, 1024
+    G = ggml.Graph()
+    Q, K, V = G.new(ggml.F32, d, t, hq, seqs), G.new(ggml.F16, d, span, hkv, seqs), G.new(ggml.F16, d, span, hkv, seqs)
+    M = G.new(ggml.F16, span, t, 1, seqs)
+    y = G.lib.ggml_flash_attn_ext(G.ctx, Q, K, V, M, d ** -0.5, 0.0, 0.0)
+    G.build(y)
+    G.allocate(gpu.buft)
+    v = RNG.integers(1, 2048, (seqs, hkv, 1, d)).astype(np.float16)
+    mask = np.where(np.arange(span) < live, 0.0, -np.inf).astype(np.float16)
+    G.set(Q, RNG.standard_normal((seqs, hq, t, d)).astype(np.float32))
+    G.set(K, np.zeros((seqs, hkv, span, d), np.float16))
+    G.set(V, np.broadcast_to(v, (seqs, hkv, span, d)))
+    G.set(M, np.broadcast_to(mask, (seqs, 1, t, span)))
+    assert G.compute(gpu.backend) == 0
+    want = np.repeat(v.astype(np.float32), hq // hkv, 1).transpose(0, 2, 1, 3)  # [seqs, 1, hq, d]
+    assert np.array_equal(G.get(y).reshape(seqs, t, hq, d), np.broadcast_to(want, (seqs, t, hq, d)))
+    G.free()
