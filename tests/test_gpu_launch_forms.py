@@ -193,11 +193,11 @@ def test_gelu_erf_against_math_erf(ggml, gpu):
 
 @pytest.mark.parametrize("heads,t,n", [(14, 390, 1), (14, 1170, 1), (3, 97, 1), (2, 64, 2), (1, 2, 3)])
 @pytest.mark.parametrize("overwritten", [False, True])
-def test_attention_over_f32_keys_and_mask(ggml, gpu, heads, t, n, overwritten):
-    """an encoder's attention over strided f32 K / V head views and a mask cast
-    from f32: the bits of the same attention over f16 tensors holding their
-    roundings. overwritten: the f32 mask changes between its cast and the
-    attention, which must not see it"""
+def test_attention_over_f32_keys(ggml, gpu, heads, t, n, overwritten):
+    """an encoder's attention over strided f32 K / V head views, its f16 mask cast
+    from f32 in the graph: the bits of the same attention over f16 tensors holding
+    their roundings. overwritten: the f32 mask changes between the cast and the
+    attention, which reads the cast's result"""
     d = 64
     print(f"f32 attention {heads} x {t} x {n} overwritten {overwritten}", flush=True)
     q, k, v = (RNG.standard_normal((n, t, heads, d)).astype(np.float32) for _ in range(3))
