@@ -232,7 +232,7 @@ __global__ __launch_bounds__(256) void k_norm(tview d, tview a, int mode, float 
 // elements a thread in one 16-byte load each of row, weight and bias, the f64
 // sums of the four waves added through LDS. Latency bound: in k_norm one wave
 // walks such a row with up to 16 four-byte loads behind exec masks and holds
-// the whole row's sums (390 rows of 896: 6.6 us there, 5.1 us here).
+// the whole row's sums (390 rows of 896: 7.4 us there, 5.2 us here).
 __global__ __launch_bounds__(256) void k_norm_row4(tview d, tview a, int mode, float eps, const float * __restrict__ wr,
                                                    const float * __restrict__ br) {
     __shared__ double s_sum[2][4];

@@ -125,9 +125,10 @@ __device__ __forceinline__ void fm_merge(float & M, float & L, float m, float l,
 //
 // KV32: K and V are f32 (the encoders' head views of their projections),
 // staged rounded to f16 -- what a copy to f16 tensors ahead of the launch
-// would hold: that launch (6.8 us a layer of a 30 s encode) goes, the
-// attention stays at 20 us. Reading an f32 mask here as well, in place of its
-// 5 us cast, measured 27.5 us: its rows on 4 bytes take a load an entry.
+// would hold: that launch (6.6 us a layer of a 30 s encode) goes, the
+// attention itself takes 21 us (23 over f16 copies, before its unmasked tiles).
+// Reading an f32 mask here as well, in place of its 5 us cast, measured 27.5 us:
+// its rows on 4 bytes take a load an entry.
 //
 // MG: the workgroup takes every split of its rows in turn and merges
 // their states in registers (fm_merge, in split order, what the combine
@@ -554,7 +555,8 @@ static int fm_q_blocks(const fattn_args & a) {
 // workgroup alone on a CU takes for a tile (at either head size). F(n) is the
 // time in which the CUs, n workgroups dealt to them, do a tile of each: with
 // heads of 128 two are resident and take 1.39 T, further ones come after them;
-// with heads of 64 two take 1.27 T, three 1.53 T, from four on 0.53 T each.
+// with heads of 64 (three resident) two take 1.27 T, three 1.53 T, from four on
+// 0.53 T each.
 // Merged, there are `blocks` workgroups of the whole span; most spans have a
 // masked tail, which these skip: 0.9 of it is counted. Split, there are
 // blocks x splits, each of a part of the span (with heads of 64 they fill the

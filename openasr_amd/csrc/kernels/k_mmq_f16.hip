@@ -33,21 +33,23 @@
 // that a wave's matrix and vector work overlap, where they ran one after the
 // other (Q4_K's scale unpacking was a branch that kept them in separate
 // blocks). 214-229 VGPRs, two workgroups a CU (174 + 88 AGPRs and one before);
-// the products above 175 -> 168, 75 -> 67 and 52 -> 51 us. A step still takes a
-// CU about twice its MFMAs' time. Wave (wr, wc) multiplies the 64 x 64 quarter (wr: rows, wc:
+// the products named below 175 -> 168, 75 -> 67 and 52 -> 51 us. A step still
+// takes a CU about four times its MFMAs' time (0.87 us against 0.21: 512 cycles
+// at 2.4 GHz). Wave (wr, wc) multiplies the 64 x 64 quarter (wr: rows, wc:
 // columns) as 4 x 4 blocks of 16 x 16: the activations are the MFMA A
 // operand (lane l: column l % 16, k 8 (l / 16) .. + 7), the weights the B
 // operand, so lane l ends with weight row l % 16 of four consecutive
 // columns and a tile's stores are 64-byte runs of an output column. Tiles
 // are dealt to the XCDs in contiguous runs (workgroup i on XCD i % 8), down
-// the row tiles of a band of four column blocks: an XCD's 32 running tiles are
-// then 8 row tiles x 4 column blocks, which walk K together and share their
-// operands' current steps in its L2. (Row tile by row tile, all column blocks
-// adjacent, they were 2 row tiles x 16 of 2048 columns: 2.6 times the distinct
-// bytes a step, and the 8 MB of activations past the 4 MB of L2, read again
-// from beyond it for every row tile.) The 1.7B layer's
-// products over 2048 columns: gate and up 181 -> 175 us, down and output 78 ->
-// 75 us on average, QKV 54 -> 52 us.
+// the row tiles of a band of four column blocks: an XCD's 64 running tiles (32
+// CUs, two each) are then 16 row tiles x 4 column blocks, which walk K together
+// and share their operands' current steps in its L2. (Row tile by row tile, all
+// column blocks adjacent, they would be 4 row tiles x 16 of 2048 columns: twice
+// the distinct bytes a step with Q4_K, and the 8 MB of activations past the
+// 4 MB of L2, read again from beyond it for every row tile.) The 1.7B layer's
+// products over 2048 columns, measured with one workgroup a CU, so 32 running
+// tiles: gate and up 181 -> 175 us, down and output 78 -> 75 us on average, QKV
+// 54 -> 52 us.
 #include <type_traits>
 
 #include "../mi355x_common.h"

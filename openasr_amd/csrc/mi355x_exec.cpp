@@ -2317,10 +2317,12 @@ static void run_steps(backend_state * be, std::vector<step> & steps, size_t firs
 }
 
 // A captured graph of at most kDirectLaunches kernels, one after the other, is
-// replayed by launching its kernels: a hipGraphLaunch costs a fixed ~25 us of
-// latency up to the end of the wait, a launch about 2.5 us and the wait 9 us.
-// Measured, launches and wait: 1 kernel 11.5 us direct, 27.2 us as a graph;
-// 2: 14.2, 29.8; 4: 18.5, 29.7; 8: 41.8, 30.6.
+// replayed by launching its kernels (from the third compute of a graph on: the
+// first runs eagerly, the second captures). Launches of an empty kernel and the
+// wait, us, direct / as a HIP graph: 1 kernel 11.5 / 27.7; 2: 14.3 / 31.6;
+// 3: 16.6 / 32.2; 4: 18.8 / 32.4; 5: 21.0 / 32.8; 6: 23.2 / 33.5; 7: 25.5 / 34.5;
+// 8: 51 / 32.2. So the line could lie at seven; of five to seven only these
+// empty kernels were measured, and the graphs gained so far have up to four.
 constexpr size_t kDirectLaunches = 4;
 
 // the kernels of a captured graph in launch order; empty when it holds more
