@@ -213,6 +213,7 @@ __device__ __forceinline__ void mmq_compute(const mmq_args & a, const mmq_slice<
 // sibling products: row_tile's product becomes the launch's (a's weights, rows
 // and output), row_tile its tile; selected with constant indices (an index
 // into the argument arrays would put them in scratch memory)
+template <bool HALF>
 __device__ __forceinline__ void mmq_pick_product(mmq_args & a, int64_t & row_tile, int tile_rows) {
     static_assert(kGemmFloatMaxSubs == 2, "product selection below");
     if (a.nsub <= 0) return;
@@ -221,14 +222,14 @@ __device__ __forceinline__ void mmq_pick_product(mmq_args & a, int64_t & row_til
     const char * sw = a.sub_W[0];
     char * sd = a.sub_dst[0];
     const float * sb = a.sub_bias[0];
-    bool sh = a.sub_f16[0];
+    bool sh = HALF && a.sub_f16[0];
     if (r0 >= a.sub_m0[1]) {
         base = a.sub_m0[1], mend = a.sub_m0[2];
-        sw = a.sub_W[1], sd = a.sub_dst[1], sb = a.sub_bias[1], sh = a.sub_f16[1];
+        sw = a.sub_W[1], sd = a.sub_dst[1], sb = a.sub_bias[1], sh = HALF && a.sub_f16[1];
     }
     if (a.nsub >= 2 && r0 >= a.sub_m0[2]) {
         base = a.sub_m0[2], mend = a.sub_m0[3];
-        sw = a.sub_W[2], sd = a.sub_dst[2], sb = a.sub_bias[2], sh = a.sub_f16[2];
+        sw = a.sub_W[2], sd = a.sub_dst[2], sb = a.sub_bias[2], sh = HALF && a.sub_f16[2];
     }
     row_tile -= base / tile_rows;
     a.M = mend - base;
@@ -239,7 +240,8 @@ __device__ __forceinline__ void mmq_pick_product(mmq_args & a, int64_t & row_til
     a.epi.f16_out = sh;
 }
 
-template <int WT, int GRPS, int RW, int KW>
+// HALF: some product's result is f16 (a branch in every store otherwise, 1-2 %)
+template <int WT, int GRPS, int RW, int KW, bool HALF>
 __global__ __launch_bounds__(64 * RW * KW) void k_mmq(mmq_args a) {
     constexpr int kRows = 16 * RW;
     __shared__ __align__(16) mmq_slice<GRPS> s_buf[2][KW];
@@ -250,9 +252,10 @@ __global__ __launch_bounds__(64 * RW * KW) void k_mmq(mmq_args a) {
     if (t >= a.tiles) return;  // before any barrier: the whole workgroup leaves
     int64_t row_tile = t / a.col_blocks;
     const int64_t col_block = t % a.col_blocks;
-    mmq_pick_product(a, row_tile, kRows);
+    mmq_pick_product<HALF>(a, row_tile, kRows);
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int rw = wave % RW, kg = wave / RW, st = (int) threadIdx.x % (64 * RW);
+    const int rw = KW > 1 ? wave % RW : wave, kg = KW > 1 ? wave / RW : 0;
+    const int st = KW > 1 ? (int) threadIdx.x % (64 * RW) : (int) threadIdx.x;
     const int r = lane & 15, g = lane >> 4;
     const int64_t row = row_tile * kRows + rw * 16 + r;
     const bool row_ok = row_tile * kRows + rw * 16 < a.M;  // uniform per wave
@@ -267,26 +270,41 @@ __global__ __launch_bounds__(64 * RW * KW) void k_mmq(mmq_args a) {
         for (int i = 0; i < 4; i++) acc[grp][i] = 0.0;
     mmq_act<GRPS, RW> act;
     wregs wn;
-    // K group kg takes the slices kg, kg + KW, ...: every group runs the same
-    // number of rounds (barriers), the groups past the last slice idle
-    if (kg < nks) {
-        mmq_act_load<WT, GRPS, RW>(a, st, n0, ncol, kg, act);
-        mmq_w_load(a, wrow, kg, g, wn);
-    }
-    int buf = 0;
-    for (int64_t k0 = 0; k0 < nks; k0 += KW, buf ^= 1) {
-        const int64_t ks = k0 + kg;
-        mmq_slice<GRPS> & S = s_buf[buf][kg];
-        if (ks < nks) mmq_act_store<WT, GRPS, RW>(a, st, ncol, ks, act, S);
-        const wregs w = wn;
-        __syncthreads();
-        if (ks + KW < nks) {
-            mmq_act_load<WT, GRPS, RW>(a, st, n0, ncol, ks + KW, act);
-            mmq_w_load(a, wrow, ks + KW, g, wn);
+    if constexpr (KW == 1) {
+        // one group: a loop of its own, as the groups' guards cost it 2-6 %
+        mmq_act_load<WT, GRPS, RW>(a, st, n0, ncol, 0, act);
+        mmq_w_load(a, wrow, 0, g, wn);
+        for (int64_t ks = 0; ks < nks; ks++) {
+            mmq_slice<GRPS> & S = s_buf[ks & 1][0];
+            mmq_act_store<WT, GRPS, RW>(a, st, ncol, ks, act, S);
+            const wregs w = wn;
+            __syncthreads();
+            if (ks + 1 < nks) {
+                mmq_act_load<WT, GRPS, RW>(a, st, n0, ncol, ks + 1, act);
+                mmq_w_load(a, wrow, ks + 1, g, wn);
+            }
+            if (row_ok) mmq_compute<GRPS>(a, S, w, ks, r, g, acc);
         }
-        if (row_ok && ks < nks) mmq_compute<GRPS>(a, S, w, ks, r, g, acc);
-    }
-    if constexpr (KW > 1) {
+    } else {
+        // K group kg takes the slices kg, kg + KW, ...: every group runs the
+        // same number of rounds (barriers), the groups past the last slice idle
+        if (kg < nks) {
+            mmq_act_load<WT, GRPS, RW>(a, st, n0, ncol, kg, act);
+            mmq_w_load(a, wrow, kg, g, wn);
+        }
+        int buf = 0;
+        for (int64_t k0 = 0; k0 < nks; k0 += KW, buf ^= 1) {
+            const int64_t ks = k0 + kg;
+            mmq_slice<GRPS> & S = s_buf[buf][kg];
+            if (ks < nks) mmq_act_store<WT, GRPS, RW>(a, st, ncol, ks, act, S);
+            const wregs w = wn;
+            __syncthreads();
+            if (ks + KW < nks) {
+                mmq_act_load<WT, GRPS, RW>(a, st, n0, ncol, ks + KW, act);
+                mmq_w_load(a, wrow, ks + KW, g, wn);
+            }
+            if (row_ok && ks < nks) mmq_compute<GRPS>(a, S, w, ks, r, g, acc);
+        }
         // the groups' sums through the staging buffers, added in group order
         double * s_acc = (double *) &s_buf[0][0];
         static_assert(sizeof(s_buf) >= sizeof(double) * 256 * GRPS * RW * (KW - 1), "the staging buffers hold the sums");
@@ -330,11 +348,14 @@ __global__ __launch_bounds__(64 * RW * KW) void k_mmq(mmq_args a) {
         for (int i = 0; i < 4; i++) {
             const int n = n0 + grp * 16 + 4 * g + i;
             if (n >= a.N) continue;
-            if (a.epi.f16_out) *(uint16_t *) (a.dst + (int64_t) n * a.dst_nb1 + row * 2) = float_to_half_bits(o[grp * 4 + i]);
+            if (HALF && a.epi.f16_out) *(uint16_t *) (a.dst + (int64_t) n * a.dst_nb1 + row * 2) = float_to_half_bits(o[grp * 4 + i]);
             else *(float *) (a.dst + (int64_t) n * a.dst_nb1 + row * 4) = o[grp * 4 + i];
         }
     }
 }
+
+template <int V>
+using mmq_int = std::integral_constant<int, V>;
 
 bool mmq_supported(int wtype, int64_t M, int64_t K) {
     if (M % 16 != 0) return false;
@@ -388,13 +409,20 @@ void launch_mmq(int wtype, const char * W, int64_t row_bytes, int64_t M, int64_t
     a.N = (int) N;
     a.dst = dst;
     a.dst_nb1 = dst_nb1;
-    auto go = [&](auto q4, auto q8, int grps, int rw, int kw) {
-        a.col_blocks = (N + 16 * grps - 1) / (16 * grps);
-        a.tiles = (m_all + 16 * rw - 1) / (16 * rw) * a.col_blocks;
+    bool half = epi.f16_out;
+    for (int i = 0; i < nsub; i++) half = half || subs[i].f16_out;
+    auto form = [&](auto grps, auto rw, auto kw) {
+        constexpr int G = decltype(grps)::value, R = decltype(rw)::value, KW = decltype(kw)::value;
+        a.col_blocks = (N + 16 * G - 1) / (16 * G);
+        a.tiles = (m_all + 16 * R - 1) / (16 * R) * a.col_blocks;
         a.per_xcd = (a.tiles + kMmqXcds - 1) / kMmqXcds;
-        const dim3 grid((unsigned) (a.per_xcd * kMmqXcds)), block((unsigned) (64 * rw * kw));
-        if (wtype == GGML_TYPE_Q4_K) hipLaunchKernelGGL(q4, grid, block, 0, stream, a);
-        else hipLaunchKernelGGL(q8, grid, block, 0, stream, a);
+        auto go = [&](auto kernel) {
+            hipLaunchKernelGGL(kernel, dim3((unsigned) (a.per_xcd * kMmqXcds)), dim3(64 * R * KW), 0, stream, a);
+        };
+        if (wtype == GGML_TYPE_Q4_K && half) go(k_mmq<GGML_TYPE_Q4_K, G, R, KW, true>);
+        else if (wtype == GGML_TYPE_Q4_K) go(k_mmq<GGML_TYPE_Q4_K, G, R, KW, false>);
+        else if (half) go(k_mmq<GGML_TYPE_Q8_0, G, R, KW, true>);
+        else go(k_mmq<GGML_TYPE_Q8_0, G, R, KW, false>);
     };
     // The form by how many 64 x 64 tiles there are for the CUs: fewer tiles,
     // more and smaller workgroups and more K groups in flight. Per call with
@@ -409,11 +437,11 @@ void launch_mmq(int wtype, const char * W, int64_t row_bytes, int64_t M, int64_t
     //   392 tiles 3584 x 896 x 390   36.7 with one group, 39.0 with two
     const int64_t tiles = (m_all + kMmqRows - 1) / kMmqRows * ((N + kMmqCols - 1) / kMmqCols);
     const bool deep = K > 512;  // slices for four K groups (K = 384: two)
-    if (deep && 6 * tiles <= n_cu) go(k_mmq<GGML_TYPE_Q4_K, 2, 1, 4>, k_mmq<GGML_TYPE_Q8_0, 2, 1, 4>, 2, 1, 4);
-    else if (deep && 4 * tiles <= n_cu) go(k_mmq<GGML_TYPE_Q4_K, 2, 2, 4>, k_mmq<GGML_TYPE_Q8_0, 2, 2, 4>, 2, 2, 4);
-    else if (4 * tiles <= 3 * n_cu) go(k_mmq<GGML_TYPE_Q4_K, 2, 2, 2>, k_mmq<GGML_TYPE_Q8_0, 2, 2, 2>, 2, 2, 2);
-    else if (tiles <= n_cu) go(k_mmq<GGML_TYPE_Q4_K, 4, 4, 2>, k_mmq<GGML_TYPE_Q8_0, 4, 4, 2>, 4, 4, 2);
-    else go(k_mmq<GGML_TYPE_Q4_K, 4, 4, 1>, k_mmq<GGML_TYPE_Q8_0, 4, 4, 1>, 4, 4, 1);
+    if (deep && 6 * tiles <= n_cu) form(mmq_int<2>{}, mmq_int<1>{}, mmq_int<4>{});
+    else if (deep && 4 * tiles <= n_cu) form(mmq_int<2>{}, mmq_int<2>{}, mmq_int<4>{});
+    else if (4 * tiles <= 3 * n_cu) form(mmq_int<2>{}, mmq_int<2>{}, mmq_int<2>{});
+    else if (tiles <= n_cu) form(mmq_int<4>{}, mmq_int<4>{}, mmq_int<2>{});
+    else form(mmq_int<4>{}, mmq_int<4>{}, mmq_int<1>{});
 }
 
 }  // namespace mi355x
