@@ -563,7 +563,10 @@ static int fm_q_blocks(const fattn_args & a) {
 // CUs evenly), and the combine and the partials cost 6 T and, with heads of
 // 128, 1/128 T a workgroup. With 64-wide heads the split form reads f32 K and V
 // itself, the merged one copies of them (8 T). So merging is refused where few
-// blocks over a long span would leave CUs idle.
+// blocks over a long span would leave CUs idle; and below a block for every
+// second CU, where the combine is small and costs less than the 6 T (one sequence
+// over 512 positions, in a row without waits: 32 queries 16.9 / 22.0, 119 19.7 /
+// 22.6, 256 22.8 / 22.3; 119 over 1000 of 1024 20.3 / 38.1).
 // Measured, us a call, split / merged (128: 16 query, 8 kv heads; queries, live
 // positions and span, sequences):
 //   128 blocks  256 q 640 of 1024, 2     44 / 38    256 q 2000 of 2048, 2    60 / 80
@@ -580,6 +583,7 @@ static int fm_q_blocks(const fattn_args & a) {
 // heads: 600 of 600, 8 (1120) 117 / 112, 1300 of 1300, 1 (294) 71 / 84. The rule
 // takes the slower form by up to 8 % at the edges (256 q 1000 of 1024, 2).
 static bool fm_merge_pays(const fattn_args & a, int64_t blocks, int n_tiles, bool kv_f32, int n_cu) {
+    if (2 * blocks < n_cu) return false;
     const bool wide = a.d == 128;
     auto shared = [&](int64_t n) {
         const double k = (double) ((n + n_cu - 1) / n_cu);
