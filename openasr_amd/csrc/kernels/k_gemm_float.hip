@@ -32,6 +32,7 @@ namespace {
 constexpr int kGfBM = 64, kGfBN = 64, kGfBK = 32;
 constexpr int kGfDepth = 4;  // slabs in flight in the aligned form (even: slab s is in LDS buffer s % 2)
 constexpr int kGfThreads = 256;
+constexpr int64_t kGfBand = 8;  // column tiles side by side in the f16-weight form's tile order
 
 typedef float gf_v4f __attribute__((ext_vector_type(4)));
 typedef _Float16 gf_v8h __attribute__((ext_vector_type(8)));
@@ -231,8 +232,7 @@ __device__ __forceinline__ void gf_as_f32(const gf_raw & v, uint4 & lo, uint4 & 
         lo = v.r[0];
         hi = v.r[1];
     }
-    lo = gf_and(lo, v.live);
-    hi = gf_and(hi, v.live);
+    if (!v.live) lo = hi = make_uint4(0, 0, 0, 0);
 }
 
 // a slab's pieces into LDS (sa, sb): f16 operands for an F16 src0 (the
@@ -297,15 +297,32 @@ __global__ __launch_bounds__(kGfThreads) void k_gemm_float_v(gemm_float_args g) 
     __shared__ __align__(16) T sb[2][kGfBN][kGfBK + PADE];
     const int tid = (int) threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    // the tile: contiguous runs of tiles a XCD; the column tiles of a row
-    // tile adjacent, then the row tiles, then the splits (or batches), so an
-    // XCD fetches a run of weight rows once, over its splits' part of K
-    const int64_t t = (int64_t) (blockIdx.x % 8) * g.per_xcd + blockIdx.x / 8;
-    if (t >= g.tiles) return;  // the grid's padding, before any barrier
-    const int64_t rt = t / g.col_blocks;
-    int64_t m0 = rt % g.row_blocks * kGfBM;
-    const int64_t n0 = t % g.col_blocks * kGfBN;
-    const int tz = (int) (rt / g.row_blocks);
+    int64_t m0, n0;
+    int tz;  // the split (one batch), or the batch
+    if constexpr (F16) {
+        // f16 weights: contiguous runs of tiles a XCD, down the row tiles of a
+        // band of kGfBand column tiles, then the bands, then the splits (or
+        // batches): an XCD's running tiles share their weight rows and columns.
+        // us, row by row over the grid / all column tiles in one band / bands of
+        // 8: 896 x 7680 x 390 43.1 / 32.2 / 32.2, 1024 x 1024 x 1000 16.3 / 14.2
+        // / 14.2, 2048 x 2048 x 2048 59.1 / 80.6 / 56.5 (the columns then pass an
+        // L2), 4096 x 1024 x 2048 61.7 / 81.7 / 58.0, 2048 x 2048 x 300 24.6 /
+        // 25.3 / 25.3; bands of 4 or 16 between
+        const int64_t t = (int64_t) (blockIdx.x % 8) * g.per_xcd + blockIdx.x / 8;
+        if (t >= g.tiles) return;  // the grid's padding, before any barrier
+        const int64_t plane = g.row_blocks * g.col_blocks, u = t % plane;
+        const int64_t band = u / (g.row_blocks * kGfBand), ub = u - band * g.row_blocks * kGfBand;
+        const int64_t left = g.col_blocks - band * kGfBand, width = left < kGfBand ? left : kGfBand;
+        m0 = ub / width * kGfBM;
+        n0 = (band * kGfBand + ub % width) * kGfBN;
+        tz = (int) (t / plane);
+    } else {
+        // f32 weights on the f32 matrix cores: in the grid's order (bound by
+        // them; XCD runs measured 896 x 3584 x 390 43.4 -> 48.8 us)
+        m0 = (int64_t) blockIdx.x * kGfBM;
+        n0 = (int64_t) blockIdx.y * kGfBN;
+        tz = (int) blockIdx.z;
+    }
     // sibling products: this tile's product (rows, weights, output, bias)
     // (selects with constant indices: an index into the argument arrays
     // would put the arguments in scratch memory)
@@ -330,7 +347,6 @@ __global__ __launch_bounds__(kGfThreads) void k_gemm_float_v(gemm_float_args g) 
         g.d_nb1 = g.M * 4;  // each product's output is contiguous
         g.epi.bias = sbias;
     }
-    // tz: the split (one batch), or the batch
     const int zb = g.splits > 1 ? 0 : tz, ks = g.splits > 1 ? tz : 0;
     const int i2 = zb % g.ne2, i3 = zb / g.ne2;
     const int64_t kb = (int64_t) ks * g.k_span;
@@ -736,7 +752,7 @@ void launch_gemm_float(const tview & d, const tview & a, int atype, const tview 
         const dim3 gv((unsigned) (g.per_xcd * 8));
         if (g.a_f16 && g.b_f16) hipLaunchKernelGGL((k_gemm_float_v<true, true>), gv, dim3(kGfThreads), 0, s, g);
         else if (g.a_f16) hipLaunchKernelGGL((k_gemm_float_v<true, false>), gv, dim3(kGfThreads), 0, s, g);
-        else if (g.b_f16) hipLaunchKernelGGL((k_gemm_float_v<false, true>), gv, dim3(kGfThreads), 0, s, g);
+        else if (g.b_f16) hipLaunchKernelGGL((k_gemm_float_v<false, true>), grid, dim3(kGfThreads), 0, s, g);
         else if (x3) {
             // one dim of tiles, dealt to the XCDs in contiguous runs
             g.tiles = (int64_t) grid.x * grid.y;
@@ -745,7 +761,7 @@ void launch_gemm_float(const tview & d, const tview & a, int atype, const tview 
             if (a_split) hipLaunchKernelGGL(k_gemm_float_x3<true>, g1, dim3(kGfThreads), 0, s, g);
             else hipLaunchKernelGGL(k_gemm_float_x3<false>, g1, dim3(kGfThreads), 0, s, g);
         }
-        else hipLaunchKernelGGL((k_gemm_float_v<false, false>), gv, dim3(kGfThreads), 0, s, g);
+        else hipLaunchKernelGGL((k_gemm_float_v<false, false>), grid, dim3(kGfThreads), 0, s, g);
         if (g.splits > 1) {
             const int64_t blocks = std::min<int64_t>((g.M * g.N + 255) / 256, 4096);
             hipLaunchKernelGGL(k_gemm_float_reduce, dim3((unsigned) blocks), dim3(256), 0, s, g);

@@ -595,3 +595,25 @@ def test_attention_divides_by_the_row_sum(ggml, gpu, d, hq, hkv, seqs, live):
     want = np.repeat(v.astype(np.float32), hq // hkv, 1).transpose(0, 2, 1, 3)  # [seqs, 1, hq, d]
     assert np.array_equal(G.get(y).reshape(seqs, t, hq, d), np.broadcast_to(want, (seqs, t, hq, d)))
     G.free()
+
+
+# bands of eight 64-column tiles: one band, a band and a remainder, several; row
+# tiles with a remainder; batches; a K that is split
+@pytest.mark.parametrize("m,k,n,b", [(200, 96, 512, 1), (200, 96, 700, 1), (64, 64, 1100, 2), (130, 1024, 600, 1)])
+def test_float_gemm_tile_bands(ggml, gpu, m, k, n, b):
+    """an f16-weight product over more column tiles than a band: every tile once"""
+    print(f"float gemm bands {m} x {k} x {n} x {b}", flush=True)
+    G = ggml.Graph()
+    W, X = G.new(ggml.F16, k, m, b, weight=True), G.new(ggml.F32, k, n, b)
+    y = G.lib.ggml_mul_mat(G.ctx, W, X)
+    G.build(y)
+    G.allocate(gpu.buft)
+    w = RNG.standard_normal((b, m, k)).astype(np.float16)
+    x = RNG.standard_normal((b, n, k)).astype(np.float32)
+    G.set(W, w), G.set(X, x)
+    assert G.compute(gpu.backend) == 0
+    want = x.astype(np.float16).astype(np.float64) @ w.astype(np.float64).transpose(0, 2, 1)
+    got = G.get(y).reshape(b, n, m)
+    # k f32 additions of products of about 1: an error below k 2^-24 each
+    assert np.abs(got - want).max() <= k * 2.0 ** -24 * np.sqrt(k) + 1e-6
+    G.free()
