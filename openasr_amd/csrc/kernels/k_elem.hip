@@ -233,6 +233,11 @@ __global__ __launch_bounds__(256) void k_norm(tview d, tview a, int mode, float 
 // sums of the four waves added through LDS. Latency bound: in k_norm one wave
 // walks such a row with up to 16 four-byte loads behind exec masks and holds
 // the whole row's sums (390 rows of 896: 7.4 us there, 5.2 us here).
+// Up to kNormRow4Rows rows: with more the CUs are full either way and a wave a
+// row moves the same bytes with a quarter of the waves (rows of 896, NORM, a wave
+// / a workgroup a row: 390 rows 5.7 / 4.3 us, 1024 6.7 / 6.0, 2048 7.5 / 7.9, 8192
+// 18.1 / 22.2).
+constexpr int64_t kNormRow4Rows = 1024;
 __global__ __launch_bounds__(256) void k_norm_row4(tview d, tview a, int mode, float eps, const float * __restrict__ wr,
                                                    const float * __restrict__ br) {
     __shared__ double s_sum[2][4];
@@ -416,7 +421,7 @@ void launch_norm(const tview & d, const tview & a, int mode, float eps, const tv
             default: hipLaunchKernelGGL((k_norm_rows<16, 4>), g1, dim3(256), 0, s, d, a, mode, eps, wp, bp, qt, ab); return;
         }
     }
-    if (a.ne[0] > 512 && a.ne[0] <= 1024 && a.ne[0] % 4 == 0 && norm_aligned(d, a, w, b)) {
+    if (rows <= kNormRow4Rows && a.ne[0] > 512 && a.ne[0] <= 1024 && a.ne[0] % 4 == 0 && norm_aligned(d, a, w, b)) {
         hipLaunchKernelGGL(k_norm_row4, dim3((unsigned) rows), dim3(256), 0, s, d, a, mode, eps,
                            w ? (const float *) w->data : nullptr, b ? (const float *) b->data : nullptr);
         return;

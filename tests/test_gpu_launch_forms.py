@@ -314,11 +314,12 @@ def test_norm_rope_rows(ggml, gpu, heads, kv_heads, t):
 
 
 @pytest.mark.parametrize("n", [512, 516, 640, 896, 1020, 1028])
-@pytest.mark.parametrize("rows", [1, 390])
+@pytest.mark.parametrize("rows", [1, 390, 1024, 1025])
 @pytest.mark.parametrize("layer", [False, True])
 def test_norm_row_widths(ggml, gpu, n, rows, layer):
     """RMS_NORM and NORM with weight and bias at the edges of the
-    workgroup-a-row form (513 to 1024 elements, a multiple of four)"""
+    workgroup-a-row form (513 to 1024 elements, a multiple of four; at most 1024
+    rows)"""
     f = np.float32
     x = (RNG.standard_normal((rows, n)) * 2 + 0.7).astype(f)
     w, b = RNG.uniform(0.5, 1.5, n).astype(f), RNG.standard_normal(n).astype(f)
