@@ -445,7 +445,8 @@ void launch_norm(const tview & d, const tview & a, int mode, float eps, const tv
 // blockIdx.y selects the job: the query and key rows of one layer share a
 // launch. A wave takes H rows (heads) of one position: the angle -- up to 63
 // multiplies in turn and a sine and cosine in double, most of the work of a
-// row -- is formed once for them.
+// row -- is formed once for them, after the rows' sums (before them, their values
+// wait in registers: 255 positions of 16 heads 5.9 us against 5.3).
 template <int H>
 __global__ __launch_bounds__(256) void k_rms_norm_rope128(norm_rope_job j0, norm_rope_job j1) {
     const norm_rope_job & j = blockIdx.y == 0 ? j0 : j1;
@@ -465,6 +466,14 @@ __global__ __launch_bounds__(256) void k_rms_norm_rope128(norm_rope_job j0, norm
     }
     const float w0 = j.w[lane], w1 = j.w[lane + 64];
     const float p = (float) j.pos[i2];
+#pragma unroll
+    for (int h = 0; h < H; h++) {
+        const double s2 = wave_sum_d((double) (x0[h] * x0[h]) + (double) (x1[h] * x1[h]));
+        const float var = (float) (s2 / 128.0);
+        const float scale = 1.0f / sqrtf(var + j.eps);
+        x0[h] = (x0[h] * scale) * w0;
+        x1[h] = (x1[h] * scale) * w1;
+    }
     float theta = p;
     for (int k = 0; k < lane; k++) theta *= j.theta_scale;
     float sn, c;
@@ -473,13 +482,9 @@ __global__ __launch_bounds__(256) void k_rms_norm_rope128(norm_rope_job j0, norm
     sn *= j.attn_factor;
 #pragma unroll
     for (int h = 0; h < H; h++) {
-        const double s2 = wave_sum_d((double) (x0[h] * x0[h]) + (double) (x1[h] * x1[h]));
-        const float var = (float) (s2 / 128.0);
-        const float scale = 1.0f / sqrtf(var + j.eps);
-        const float v0 = (x0[h] * scale) * w0, v1 = (x1[h] * scale) * w1;
         float * yh = (float *) ((char *) y + h * j.d.nb[1]);
-        yh[lane] = v0 * c - v1 * sn;
-        yh[lane + 64] = v0 * sn + v1 * c;
+        yh[lane] = x0[h] * c - x1[h] * sn;
+        yh[lane + 64] = x0[h] * sn + x1[h] * c;
     }
 }
 
