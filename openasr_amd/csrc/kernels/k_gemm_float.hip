@@ -32,7 +32,7 @@ namespace {
 constexpr int kGfBM = 64, kGfBN = 64, kGfBK = 32;
 constexpr int kGfDepth = 4;  // slabs in flight in the aligned form (even: slab s is in LDS buffer s % 2)
 constexpr int kGfThreads = 256;
-constexpr int64_t kGfBand = 8;  // column tiles side by side in the f16-weight form's tile order
+constexpr uint32_t kGfBand = 8;  // column tiles side by side in the f16-weight form's tile order
 
 typedef float gf_v4f __attribute__((ext_vector_type(4)));
 typedef _Float16 gf_v8h __attribute__((ext_vector_type(8)));
@@ -308,14 +308,17 @@ __global__ __launch_bounds__(kGfThreads) void k_gemm_float_v(gemm_float_args g) 
         // / 14.2, 2048 x 2048 x 2048 59.1 / 80.6 / 56.5 (the columns then pass an
         // L2), 4096 x 1024 x 2048 61.7 / 81.7 / 58.0, 2048 x 2048 x 300 24.6 /
         // 25.3 / 25.3; bands of 4 or 16 between
-        const int64_t t = (int64_t) (blockIdx.x % 8) * g.per_xcd + blockIdx.x / 8;
-        if (t >= g.tiles) return;  // the grid's padding, before any barrier
-        const int64_t plane = g.row_blocks * g.col_blocks, u = t % plane;
-        const int64_t band = u / (g.row_blocks * kGfBand), ub = u - band * g.row_blocks * kGfBand;
-        const int64_t left = g.col_blocks - band * kGfBand, width = left < kGfBand ? left : kGfBand;
-        m0 = ub / width * kGfBM;
-        n0 = (band * kGfBand + ub % width) * kGfBN;
-        tz = (int) (t / plane);
+        // (a grid's workgroups: 32 bits, whose divisions a short launch feels)
+        const uint32_t t = blockIdx.x % 8 * (uint32_t) g.per_xcd + blockIdx.x / 8;
+        if (t >= (uint32_t) g.tiles) return;  // the grid's padding, before any barrier
+        const uint32_t rows = (uint32_t) g.row_blocks, cols = (uint32_t) g.col_blocks;
+        const uint32_t z = t / (rows * cols), u = t - z * (rows * cols);
+        const uint32_t band = u / (rows * kGfBand), ub = u - band * rows * kGfBand;
+        const uint32_t left = cols - band * kGfBand, width = left < kGfBand ? left : kGfBand;
+        const uint32_t rb = ub / width;
+        m0 = (int64_t) rb * kGfBM;
+        n0 = (int64_t) (band * kGfBand + (ub - rb * width)) * kGfBN;
+        tz = (int) z;
     } else {
         // f32 weights on the f32 matrix cores: in the grid's order (bound by
         // them; XCD runs measured 896 x 3584 x 390 43.4 -> 48.8 us)
